@@ -532,34 +532,50 @@ __device__ __forceinline__ typename MetricOf<GEOM>::type metric_at(const DevPara
 }
 
 // ---- bounds: fixup.hpp:91-134, 188-213 ------------------------------------------------
-__device__ __forceinline__ void get_floors(const DevBounds &b, double x1, double x2,
-                                           double x3, double &rflr, double &sflr) {
+// GetFloors at a point, in two parts: what depends on the position alone (exp and pow of the
+// profiles), evaluated once per zone or face, and the specific-energy floor for a given
+// density, which depends on that density for EXPX1_RHO_U only.  The inversion evaluates its
+// floor at every step of the root find: with the profiles inside that loop each of the five
+// places that need a floor carried the whole profile switch (pow included): the fused update
+// was 65 KB of code and is 28 KB now, and an FMKS torus zone took two exp per residual
+// evaluation (2^22 Kerr-Schild states 535 -> 458 us together with the conditional store of
+// k_con2prim_batch; a 150 x 90 x 70 hydro stage 264 -> 231 us with the MHD-free residual).
+struct Floors {
+  double rho;  // the density floor
+  double sie;  // the specific-energy floor (EXPX1_RHO_U: its numerator, the energy-density floor)
+  double den;  // EXPX1_RHO_U: the density floor before the EOS minimum
+};
+__device__ __forceinline__ Floors floors_at(const DevBounds &b, double x1, double x2,
+                                            double x3) {
+  Floors f;
+  f.den = 0.0;
   switch (b.floor_type) {
   case PHX_FLOOR_CONSTANT_RHO_SIE:
-    rflr = b.r0;
-    sflr = b.s0;
+    f.rho = b.r0;
+    f.sie = b.s0;
     break;
   case PHX_FLOOR_EXPX1_RHO_SIE:
-    rflr = b.r0 * exp(b.ralpha * x1);
-    sflr = b.s0 * exp(b.salpha * x1);
-    break;
-  case PHX_FLOOR_EXPX1_RHO_U: {
-    const double scratch = b.r0 * exp(b.ralpha * x1);
-    sflr = b.s0 * exp(b.salpha * x1) / smax(rflr, scratch);
-    rflr = scratch;
-  } break;
-  case PHX_FLOOR_X1_RHO_SIE:
-    rflr = b.r0 * smin(1.0, pow(x1, b.ralpha));
-    sflr = b.s0 * smin(1.0, pow(x1, b.salpha));
+  case PHX_FLOOR_EXPX1_RHO_U:
+    f.rho = b.r0 * exp(b.ralpha * x1);
+    f.sie = b.s0 * exp(b.salpha * x1);
+    f.den = f.rho;
     break;
   default: {
-    const double r = sqrt(x1 * x1 + x2 * x2 + x3 * x3);
-    rflr = b.r0 * smin(1.0, pow(r, b.ralpha));
-    sflr = b.s0 * smin(1.0, pow(r, b.salpha));
+    // X1_RHO_SIE scales with x1, R_RHO_SIE with the Cartesian radius
+    const double r =
+        b.floor_type == PHX_FLOOR_X1_RHO_SIE ? x1 : sqrt(x1 * x1 + x2 * x2 + x3 * x3);
+    f.rho = b.r0 * smin(1.0, pow(r, b.ralpha));
+    f.sie = b.s0 * smin(1.0, pow(r, b.salpha));
   } break;
   }
-  rflr = smax(rflr, b.rho_min_eos);
-  sflr = smax(sflr, b.sie_min_eos);
+  f.rho = smax(f.rho, b.rho_min_eos);
+  if (b.floor_type != PHX_FLOOR_EXPX1_RHO_U) f.sie = smax(f.sie, b.sie_min_eos);
+  return f;
+}
+__device__ __forceinline__ double sie_floor_of(const DevBounds &b, const Floors &f, double rho) {
+  return b.floor_type == PHX_FLOOR_EXPX1_RHO_U
+             ? smax(f.sie / smax(rho, f.den), b.sie_min_eos)
+             : f.sie;
 }
 
 // ---- ideal-gas EOS (singularity-eos IdealGas closed forms, unit scales 1) -------------
@@ -587,13 +603,12 @@ struct Layout {
 // ---- riemann.hpp:88-209 FluxState::prim_to_flux (Valencia energy) ---------------------
 template <bool MHD, class M>
 __device__ __forceinline__ void prim_to_flux(const DevParams &p, const int dir, const M &g,
-                                             const double X[3], const double *q,
+                                             const Floors &fl, const double *q,
                                              double &vm, double &vp, double *U, double *F) {
   using L = Layout<MHD>;
-  double rho_floor = q[0], sie_floor;
-  get_floors(p.bnd, X[0], X[1], X[2], rho_floor, sie_floor);
+  const double sie_floor = sie_floor_of(p.bnd, fl, q[0]);
   const double gam_max = p.bnd.gam_max, sie_max = p.bnd.sie_max;
-  const double rho = smax(q[0], rho_floor);
+  const double rho = smax(q[0], fl.rho);
   double vpcon[3] = {q[1], q[2], q[3]};
   double vsq0 = 0.;
 #pragma unroll
@@ -698,8 +713,9 @@ __device__ __forceinline__ double riemann_flux(const DevParams &p, int dir, cons
                                                const double *qr, double *flux) {
   constexpr int NC = Layout<MHD>::ncons;
   double Ul[NC], Ur[NC], Fl[NC], Fr[NC], vml, vpl, vmr, vpr;
-  prim_to_flux<MHD>(p, dir, g, X, ql, vml, vpl, Ul, Fl);
-  prim_to_flux<MHD>(p, dir, g, X, qr, vmr, vpr, Ur, Fr);
+  const Floors fl = floors_at(p.bnd, X[0], X[1], X[2]);  // one point for both states
+  prim_to_flux<MHD>(p, dir, g, fl, ql, vml, vpl, Ul, Fl);
+  prim_to_flux<MHD>(p, dir, g, fl, qr, vmr, vpr, Ur, Fr);
   if constexpr (RIEMANN == PHX_RIEMANN_LLF) {
     const double cmax = smax(smax(-vml, vpl), smax(-vmr, vpr));
 #pragma unroll
@@ -798,18 +814,24 @@ __device__ __forceinline__ void p2c(const double rho, const double vp[3], const 
 }
 
 // ---- con2prim_robust.hpp:46-180 Residual ----------------------------------------------
+// Without a magnetic field (MHD = false) b^2 and (r.b)^2 are exact zeros, so x = 1/(1 + 0),
+// rbar^2 = r^2 and qbar = q to the bit: a division and nine operations less per evaluation.
+template <bool MHD>
 struct Residual {
   const DevParams *p;
   double D, q, bsq, bsq_rpsq, rsq, rbsq, v0sq;
-  double x1, x2, x3;
-  double rho_floor, e_floor, e_max;
+  Floors fl;  // sie scaled by c2p_floor_scale_fac where it does not depend on the density
+  double rho_floor, e_max;
   bool used_density_floor, used_energy_floor, used_energy_max, used_gamma_max;
 
-  __device__ __forceinline__ double x_mu(double mu) const { return ratio(1.0, 1.0 + mu * bsq); }
+  __device__ __forceinline__ double x_mu(double mu) const {
+    return MHD ? ratio(1.0, 1.0 + mu * bsq) : 1.0;
+  }
   __device__ __forceinline__ double rbarsq_mu(double mu, double x) const {
-    return x * (x * rsq + mu * (1.0 + x) * rbsq);
+    return MHD ? x * (x * rsq + mu * (1.0 + x) * rbsq) : rsq;
   }
   __device__ __forceinline__ double qbar_mu(double mu, double x) const {
+    if constexpr (!MHD) return q;
     const double mux = mu * x;
     return q - 0.5 * (bsq + mux * mux * bsq_rpsq);
   }
@@ -825,9 +847,10 @@ struct Residual {
   }
   __device__ __forceinline__ double ehat_mu(double mu, double qbar, double rbarsq,
                                             double vhatsq, double What) {
-    double rho = rhohat_mu(ratio(1.0, What));
-    get_floors(p->bnd, x1, x2, x3, rho, e_floor);
-    e_floor *= p->fsf;
+    const double rho = rhohat_mu(ratio(1.0, What));
+    const double e_floor = p->bnd.floor_type == PHX_FLOOR_EXPX1_RHO_U
+                               ? sie_floor_of(p->bnd, fl, rho) * p->fsf
+                               : fl.sie;
     const double ehat_trial =
         What * (qbar - mu * rbarsq) + vhatsq * What * ratio(What, 1.0 + What);
     used_energy_floor = false;
@@ -975,20 +998,21 @@ __device__ __forceinline__ double regula_falsi_bracketed(F &f, double a, double 
 // con2prim_robust.hpp:299-453 for one zone, in three pieces so that a bracket predictor
 // can run between the set-up and the root find: c2p_setup (:303-367), the root find
 // (:374-376), c2p_unwrap (:382-452).
+template <bool MHD>
 struct C2PState {
-  Residual res;
+  Residual<MHD> res;
   double rcon[3], bu[3], bdotr;
 };
 
 // :303-367.  Returns false for the NaN early-out (the zone keeps every field).
 template <bool MHD, class M>
 __device__ __forceinline__ bool c2p_setup(const DevParams &p, const M &g, const double X[3],
-                                          const double *cons, double *prim, C2PState &z) {
+                                          const double *cons, double *prim,
+                                          C2PState<MHD> &z) {
   if (isnan(cons[0]) + isnan(cons[1]) + isnan(cons[4]) > 0) return false;
   const double igdet = 1.0 / g.detgamma();
-  double rhoflr = 0.0, epsflr;
-  get_floors(p.bnd, X[0], X[1], X[2], rhoflr, epsflr);
-  rhoflr *= p.fsf;
+  Floors fl = floors_at(p.bnd, X[0], X[1], X[2]);
+  const double rhoflr = fl.rho * p.fsf;
   const double gam_max = p.bnd.gam_max;
   const double D = cons[0] * igdet;
   const double tau = cons[4] * igdet;
@@ -1027,29 +1051,25 @@ __device__ __forceinline__ bool c2p_setup(const DevParams &p, const M &g, const 
   z.bdotr = bdotr;
   const double zsq = rsq / 1.0;
   const double v0sq = smin(zsq / (1.0 + zsq), 1.0 - 1.0 / (gam_max * gam_max));
-  Residual &res = z.res;
+  Residual<MHD> &res = z.res;
   res.p = &p;
   res.D = D; res.q = q; res.bsq = bsq; res.bsq_rpsq = bsq_rpsq; res.rsq = rsq;
-  res.rbsq = rbsq; res.v0sq = v0sq; res.x1 = X[0]; res.x2 = X[1]; res.x3 = X[2];
-  {
-    double garbage = 0.0;
-    res.rho_floor = 0.0;
-    get_floors(p.bnd, X[0], X[1], X[2], res.rho_floor, garbage);
-    res.e_max = p.bnd.sie_max;
-    res.rho_floor *= p.fsf;
-  }
-  res.e_floor = 0.0;
+  res.rbsq = rbsq; res.v0sq = v0sq;
+  res.rho_floor = rhoflr;
+  res.e_max = p.bnd.sie_max;
+  if (p.bnd.floor_type != PHX_FLOOR_EXPX1_RHO_U) fl.sie *= p.fsf;
+  res.fl = fl;
   res.used_density_floor = res.used_energy_floor = res.used_energy_max = res.used_gamma_max = false;
   return true;
 }
 
 // :382-452 after the root mu; returns the fail-flag value
 template <bool MHD, class M>
-__device__ __forceinline__ double c2p_unwrap(const DevParams &p, const M &g, C2PState &z,
+__device__ __forceinline__ double c2p_unwrap(const DevParams &p, const M &g, C2PState<MHD> &z,
                                              const double mu, double *cons, double *prim,
                                              double &temp, double sig[3]) {
   using L = Layout<MHD>;
-  Residual &res = z.res;
+  Residual<MHD> &res = z.res;
   const double x = res.x_mu(mu);
   const double rbarsq = res.rbarsq_mu(mu, x);
   const double vsq = res.vhatsq_mu(mu, rbarsq);
@@ -1106,14 +1126,16 @@ __device__ __forceinline__ double c2p_unwrap(const DevParams &p, const M &g, C2P
 }
 
 // the whole solve with the reference's root find: regula_falsi on [0, 1] split at the
-// guess mu_io.  iters = -1 marks an unbracketed root.
+// guess mu_io.  iters = -1 marks an unbracketed root; rederived tells whether a floor or
+// ceiling changed cons.
 template <bool MHD, class M>
 __device__ __forceinline__ double con2prim_zone(const DevParams &p, const M &g,
                                                 const double X[3], double *cons,
                                                 double *prim, double &temp, double &mu_io,
-                                                double sig[3], int &iters) {
+                                                double sig[3], int &iters, bool &rederived) {
   iters = 0;
-  C2PState z;
+  rederived = false;
+  C2PState<MHD> z;
   if (!c2p_setup<MHD>(p, g, X, cons, prim, z)) return 0.0;
   double mu;
   if (!regula_falsi(z.res, 0.0, 1.0, p.tol, mu_io, p.max_iter, mu, iters)) {
@@ -1121,7 +1143,10 @@ __device__ __forceinline__ double con2prim_zone(const DevParams &p, const M &g,
     return 0.0;
   }
   mu_io = mu;
-  return c2p_unwrap<MHD>(p, g, z, mu, cons, prim, temp, sig);
+  const double st = c2p_unwrap<MHD>(p, g, z, mu, cons, prim, temp, sig);
+  rederived = z.res.used_density_floor || z.res.used_energy_floor || z.res.used_energy_max ||
+              z.res.used_gamma_max;
+  return st;
 }
 
 // con2prim_zone on a zone's fields in memory (component planes, cell c; the zone-centre
@@ -1144,7 +1169,7 @@ __device__ __forceinline__ double con2prim_fields(const DevParams &p, const Bloc
   using M = typename MetricOf<GEOM>::type;
   using L = Layout<MHD>;
   iters = 0;
-  C2PState z;
+  C2PState<MHD> z;
   double pr[L::nprim];
   const M g = metric_at<GEOM, CACHED>(p, b, 0, q, X[0], X[1], X[2]);
   c2p_setup<MHD>(p, g, X, cs, pr, z);

@@ -146,8 +146,8 @@ __device__ __forceinline__ bool floors_needed(const DevParams &p, const DevFixup
   using M = typename MetricOf<GEOM>::type;
   const long c = ((long)k * b.nj + j) * b.ni + i;
   const double X[3] = {xc(b, 0, i), xc(b, 1, j), xc(b, 2, k)};
-  double rho_floor, sie_floor;
-  get_floors(p.bnd, X[0], X[1], X[2], rho_floor, sie_floor);
+  const Floors fl = floors_at(p.bnd, X[0], X[1], X[2]);
+  const double rho_floor = fl.rho, sie_floor = sie_floor_of(p.bnd, fl, 0.0);
   const M g = metric_at<GEOM, CACHED>(p, b, 0, (long)j * b.ni + i, X[0], X[1], X[2]);
   double pr[8];
 #pragma unroll
@@ -170,8 +170,8 @@ __device__ __forceinline__ void floors_cell(const DevParams &p, const DevFixup &
   const long n = b.ncell;
   const long c = ((long)k * b.nj + j) * b.ni + i;
   const double X[3] = {xc(b, 0, i), xc(b, 1, j), xc(b, 2, k)};
-  double rho_floor, sie_floor;
-  get_floors(p.bnd, X[0], X[1], X[2], rho_floor, sie_floor);
+  const Floors fl = floors_at(p.bnd, X[0], X[1], X[2]);
+  const double rho_floor = fl.rho, sie_floor = sie_floor_of(p.bnd, fl, 0.0);
   const double gamma_max = p.bnd.gam_max, e_max = p.bnd.sie_max;
   const M g = metric_at<GEOM, CACHED>(p, b, 0, (long)j * b.ni + i, X[0], X[1], X[2]);
   double pr[L::nprim];
@@ -211,7 +211,8 @@ __device__ __forceinline__ void floors_cell(const DevParams &p, const DevFixup &
     for (int d = 0; d < 3; ++d) sig[d] = d < b.ndim ? csig[d * n + c] : 0.0;
     double m_io = mu[c];
     int it = 0;
-    const double status = con2prim_zone<MHD>(p, g, X, cs, pr, t, m_io, sig, it);
+    bool rederived;
+    const double status = con2prim_zone<MHD>(p, g, X, cs, pr, t, m_io, sig, it, rederived);
     mu[c] = m_io;
     for (int d = 0; d < b.ndim; ++d) csig[d * n + c] = sig[d];
     if (status == 0.0) {  // :473-497

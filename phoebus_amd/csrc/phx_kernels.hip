@@ -544,9 +544,14 @@ __global__ __launch_bounds__(256) void k_con2prim_batch(DevParams p, long n,
   for (int v = 0; v < L::nprim; ++v) pr[v] = 0.0;
   double tt = 0.0, m = mu[s];
   int it = 0;
-  const double st = con2prim_zone<MHD>(p, g, X, cs, pr, tt, m, sig, it);
+  bool rederived;
+  const double st = con2prim_zone<MHD>(p, g, X, cs, pr, tt, m, sig, it, rederived);
+  // the conserved state goes back only where a floor or ceiling re-derived it: stored for
+  // every state it was 40 of the 224 bytes a state moves
+  if (rederived) {
 #pragma unroll
-  for (int v = 0; v < 5; ++v) cons[v * n + s] = cs[v];
+    for (int v = 0; v < 5; ++v) cons[v * n + s] = cs[v];
+  }
 #pragma unroll
   for (int v = 0; v < L::nprim; ++v) prim[v * n + s] = pr[v];
   mu[s] = m;

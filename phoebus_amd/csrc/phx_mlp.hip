@@ -234,7 +234,9 @@ __device__ __forceinline__ f32x4 mlp_tile_forward(const MlpDev &m, const Split &
 }
 
 // standardized features of one zone from its con2prim set-up
-__device__ __forceinline__ void zone_features(const MlpDev &m, const Residual &r, float f[4]) {
+template <bool MHD>
+__device__ __forceinline__ void zone_features(const MlpDev &m, const Residual<MHD> &r,
+                                              float f[4]) {
   const double raw[4] = {log(fmax(r.q, 0.0) + 1e-12), log(fmax(r.rsq, 0.0) + 1e-12),
                          log(fmax(r.bsq, 0.0) + 1e-12), log(fmax(r.rbsq, 0.0) + 1e-24)};
 #pragma unroll
@@ -599,7 +601,7 @@ __attribute__((amdgpu_waves_per_eu(3))) void k_con2prim_batch_learned(
       double cs[L::ncons], pr[L::nprim];
 #pragma unroll
       for (int v = 0; v < L::ncons; ++v) cs[v] = cons[v * n + sc];
-      C2PState z;
+      C2PState<MHD> z;
       if (c2p_setup<MHD>(p, g, X, cs, pr, z)) zone_features(ml, z.res, f);
     }
     // phase 2: the network for the wave's 64 states
@@ -622,10 +624,11 @@ __attribute__((amdgpu_waves_per_eu(3))) void k_con2prim_batch_learned(
     for (int v = 0; v < L::ncons; ++v) cs[v] = cin[v * n + sc];
 #pragma unroll
     for (int v = 0; v < L::nprim; ++v) pr[v] = 0.0;
-    C2PState z;
+    C2PState<MHD> z;
     const bool ok = c2p_setup<MHD>(p, g, X, cs, pr, z);
     double st = 0.0, root = mu[s], tt = 0.0;
     int it = 0, ev = 0, fb = 0;
+    bool rederived = false;
     if (ok) {
       const double c = exp((double)o1) / (double)prior_z0(ml, f[0], f[2]);
       const double w = c * fmax((double)ml.width_scale * exp((double)o2), (double)ml.width_min);
@@ -645,10 +648,14 @@ __attribute__((amdgpu_waves_per_eu(3))) void k_con2prim_batch_learned(
       if (good) {
         ev += it;
         st = c2p_unwrap<MHD>(p, g, z, root, cs, pr, tt, sig);
+        rederived = z.res.used_density_floor || z.res.used_energy_floor ||
+                    z.res.used_energy_max || z.res.used_gamma_max;
       }
     }
+    if (rederived) {
 #pragma unroll
-    for (int v = 0; v < 5; ++v) cons[v * n + s] = cs[v];
+      for (int v = 0; v < 5; ++v) cons[v * n + s] = cs[v];
+    }
 #pragma unroll
     for (int v = 0; v < L::nprim; ++v) prim[v * n + s] = pr[v];
     mu[s] = root;
@@ -712,7 +719,7 @@ k_pack_con2prim_cold(DevParams p, MlpDev m, PackView v, ColdQueue q,
       double cs[L::ncons], pr[L::nprim];
 #pragma unroll
       for (int t = 0; t < L::ncons; ++t) cs[t] = E.u_out[t * n + c];
-      C2PState z;
+      C2PState<true> z;
       if (c2p_setup<true>(p, gm, X, cs, pr, z)) zone_features(ml, z.res, f);
     }
     // phase 2: the network for the wave's 64 cells
@@ -752,7 +759,7 @@ k_pack_con2prim_cold(DevParams p, MlpDev m, PackView v, ColdQueue q,
 #pragma unroll
     for (int t = 0; t < L::nprim; ++t) pr[t] = prim[t * n + c];
     double tt = E.temp ? E.temp[c] : 0.0, root = E.mu[c];
-    C2PState z;
+    C2PState<true> z;
     c2p_setup<true>(p, gm, X, cs, pr, z);
     const double cc = exp((double)o1) / (double)prior_z0(ml, f[0], f[2]);
     const double wd = cc * fmax((double)ml.width_scale * exp((double)o2), (double)ml.width_min);
@@ -812,7 +819,7 @@ __global__ __launch_bounds__(256) void k_c2p_features(DevParams p, MlpDev m, lon
   double cs[L::ncons], pr[L::nprim];
 #pragma unroll
   for (int v = 0; v < L::ncons; ++v) cs[v] = cons[v * n + s];
-  C2PState z;
+  C2PState<MHD> z;
   float f[4] = {0.f, 0.f, 0.f, 0.f};
   if (c2p_setup<MHD>(p, g, X, cs, pr, z)) zone_features(m, z.res, f);
   for (int i = 0; i < 4; ++i) feat[i * n + s] = f[i];

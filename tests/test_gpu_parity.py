@@ -170,6 +170,46 @@ def test_batch_p2c_c2p_parity(phx, geom, mhd):
     assert relerr(prim_g[0], prims[0]) < 1e-6
 
 
+@pytest.mark.parametrize("mhd", [False, True])
+@pytest.mark.parametrize("ftype", [A.FLOOR_CONSTANT_RHO_SIE, A.FLOOR_EXPX1_RHO_SIE,
+                                   A.FLOOR_EXPX1_RHO_U, A.FLOOR_X1_RHO_SIE, A.FLOOR_R_RHO_SIE])
+def test_batch_floor_profiles(phx, ftype, mhd):
+    """Every floor profile, acting on about half of the states: flags as the oracle's, roots
+    within 4 tol and primitives within 1e-7 (both solvers stop anywhere in a bracket of
+    half-width tol; exp and pow differ by an ulp from glibc's), and the conserved state
+    rewritten exactly where a floor re-derived it."""
+    say(f"[gpu] batch floors type={ftype} mhd={mhd}")
+    n = 1023
+    rng = np.random.default_rng(40 + ftype)
+    gamma = 5.0 / 3.0
+    prims = np.ascontiguousarray(PH.random_prims(rng, n, mhd, gamma, wmax=2.0))
+    coords = np.ascontiguousarray(rng.uniform(1.0, 2.0, (2, n)))
+    rho0, sie0 = np.median(prims[0]), np.median(prims[4] / prims[0])
+    if ftype == A.FLOOR_EXPX1_RHO_U:
+        sie0 *= rho0
+    p = fluid_params(gamma=gamma, mhd=mhd, c2p_tol=1e-10, floor_scale_fac=0.5, ceilings=(50.0, 50.0),
+                     floors=dict(floor_type=ftype, rho0=rho0, sie0=sie0, rho_exp=-0.5, sie_exp=-0.25,
+                                 rho_min_eos=1e-10, sie_min_eos=1e-10))
+    op = oparams(p)
+    cons = O.p2c_batch(op, coords, prims)
+    ref = O.c2p_batch(op, coords, cons)
+    d_cons, d_coords = DeviceArray.from_host(cons), DeviceArray.from_host(coords)
+    d_prim, d_mu = DeviceArray(ref["prim"].shape), DeviceArray.from_host(np.zeros(n))
+    d_fail = DeviceArray((n,))
+    phx.con2prim_batch(p, n, d_coords, d_cons, d_prim, d_mu, d_fail)
+    synchronize()
+    assert np.array_equal(d_fail.get(), ref["fail"])
+    assert np.max(np.abs(d_mu.get() - ref["mu"])) <= 4 * p.c2p_tol
+    scale = np.maximum(np.abs(ref["prim"]), np.max(np.abs(ref["prim"][1:4]), axis=0))
+    assert np.all(np.abs(d_prim.get() - ref["prim"]) <= 1e-7 * scale)
+    out = d_cons.get()
+    changed = np.any(ref["cons"][:5] != cons[:5], axis=0)
+    assert 0.05 * n < changed.sum() < 0.95 * n
+    assert np.array_equal(np.any(out[:5] != cons[:5], axis=0), changed)
+    cscale = np.max(np.abs(ref["cons"][:5]), axis=0)
+    assert np.all(np.abs(out[:5] - ref["cons"][:5]) <= 1e-7 * cscale)
+
+
 def test_batch_edge_sizes(phx):
     # an empty batch is a no-op (no pointer is read), a negative one is refused, and ragged
     # sizes (not multiples of a wave or a 256-lane group) match the oracle bit for bit and
