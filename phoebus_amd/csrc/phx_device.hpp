@@ -36,6 +36,7 @@ struct DevParams {
     int derefine_poles;
     double h, xt, alpha, x0, smooth, hexp_br, hexp_nsq, hexp_csq, norm;
   } mgr;
+  double vsq_max;  // 1 - 1 / gam_max^2
   double fd_eps;  // eps^(1/3), the finite-difference scale of the FMKS derivatives
 };
 
@@ -120,6 +121,44 @@ __device__ __forceinline__ double xf(const BlockGeom &b, int d, int idx) {
   return b.xmin[d] + (idx - b.istart[d]) * b.dx[d];
 }
 
+// ---- correctly rounded division and square root -----------------------------------------
+// The quotient and the root in the iterations of Markstein (IBM J. Res. Develop. 34 (1990)
+// 111-119): the hardware estimate refined by two Newton steps, then the quotient corrected by
+// its exact remainder.  They give the IEEE results wherever no intermediate leaves the normal
+// range (|b| and |a / b| within 2^+-960, |a| above 2^-900 or zero; compared with the
+// compiler's a / b and sqrt on 2^24 operands with exponents within +-380 and +-900), and
+// div_fixup / the class test give the special cases (zeros, infinities, NaN).  The
+// compiler's sequences also scale operands near the ends of the range, which nothing in
+// the fluid path reaches: 70 and 90 issue cycles of a SIMD per wave against 56 and 66 here, and a
+// further quotient by the same denominator costs 18 (its reciprocal is one common
+// subexpression).  The sweeps of the exact arithmetic spend a fifth of their instructions in
+// divisions and the root find half of its time.
+__device__ __forceinline__ double refined_rcp(double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = fma(fma(-b, y, 1.0), y, y);
+  return fma(fma(-b, y, 1.0), y, y);
+}
+__device__ __forceinline__ double ddiv(double a, double b) {
+  const double y = refined_rcp(b), q = a * y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-b, q, a), y, q), b, a);
+}
+// for a denominator that is never zero where the quotient matters (no fixup; an infinite one
+// gives NaN)
+__device__ __forceinline__ double ddiv_normal(double a, double b) {
+  const double y = refined_rcp(b), q = a * y;
+  return fma(fma(-b, q, a), y, q);
+}
+__device__ __forceinline__ double dsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  g = fma(fma(-g, g, x), h, g);
+  return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +-0 and +inf are their own roots
+}
+
 // ---- robust.hpp:10-40 -------------------------------------------------------------------
 constexpr double kSmall = 10.0 * DBL_MIN;
 constexpr double kEps = 10.0 * DBL_EPSILON;
@@ -127,7 +166,7 @@ __device__ __forceinline__ double smin(double a, double b) { return (b < a) ? b 
 __device__ __forceinline__ double smax(double a, double b) { return (a < b) ? b : a; }
 __device__ __forceinline__ double ratio(double a, double b) {
   const double sgn = b >= 0 ? 1.0 : -1.0;
-  return a / (b + sgn * kSmall);
+  return ddiv(a, b + sgn * kSmall);
 }
 __device__ __forceinline__ double make_positive(double v) { return smax(v, kEps); }
 __device__ __forceinline__ double make_bounded(double v, double lo, double hi) {
@@ -136,8 +175,8 @@ __device__ __forceinline__ double make_bounded(double v, double lo, double hi) {
 
 // ---- arithmetic of the face states and fluxes ------------------------------------------
 // The reconstruction, prim_to_flux and the Riemann solvers divide and take square roots
-// through these.  By default they are IEEE division and sqrt, which round exactly as the
-// reference.  A translation unit that defines PHX_FLUX_FAST as 1 (the sweeps of the fast
+// through these.  By default they are the correctly rounded division and root above, as
+// the reference's.  A translation unit that defines PHX_FLUX_FAST as 1 (the sweeps of the fast
 // flux arithmetic, phx_flux_fast.hip, also built with contraction on) gets reciprocals and
 // reciprocal square roots from the hardware estimates (v_rcp_f64, v_rsq_f64, 24 bits)
 // refined by one Newton-Raphson step (Markstein, IBM J. Res. Develop. 34 (1990) 111-119),
@@ -159,14 +198,22 @@ __device__ __forceinline__ double frcp(double b) {
     const double r = __builtin_amdgcn_rcp(b);
     return fma(fma(-b, r, 1.0), r, r);
   } else {
-    return 1.0 / b;
+    return ddiv(1.0, b);
   }
 }
 __device__ __forceinline__ double fdiv(double a, double b) {
   if constexpr (kFluxFast)
     return a * frcp(b);
   else
-    return a / b;
+    return ddiv(a, b);
+}
+// fdiv where the denominator is positive and finite (the WENO weights: an infinite
+// smoothness indicator makes the edge NaN with either)
+__device__ __forceinline__ double fdiv_normal(double a, double b) {
+  if constexpr (kFluxFast)
+    return a * frcp(b);
+  else
+    return ddiv_normal(a, b);
 }
 // 1 / sqrt(x): y <- y + y (1 - x y^2) / 2 (v_rsq_f64: 2^-24.2; one step: 4.3e-15)
 __device__ __forceinline__ double frsqrt(double x) {
@@ -174,7 +221,7 @@ __device__ __forceinline__ double frsqrt(double x) {
     const double y = __builtin_amdgcn_rsq(x);
     return fma(0.5 * y, fma(-x * y, y, 1.0), y);
   } else {
-    return 1.0 / sqrt(x);
+    return ddiv(1.0, dsqrt(x));
   }
 }
 // sqrt(x): s = x y from the estimate y of 1/sqrt(x), then s <- s + y (x - s^2) / 2
@@ -184,7 +231,7 @@ __device__ __forceinline__ double fsqrt(double x) {
     const double s = x * y;
     return fma(0.5 * y, fma(-s, s, x), s);
   } else {
-    return sqrt(x);
+    return dsqrt(x);
   }
 }
 // robust::ratio with the flux arithmetic
@@ -227,12 +274,12 @@ __device__ __forceinline__ void recon_weno5z(double q0, double q1, double q2, do
   b = q4 - 4.0 * q3 + 3.0 * q2;
   double beta2 = tt * a * a + b * b + eps;
   const double tau5 = fabs(beta2 - beta0);
-  beta0 = fdiv(beta0 + tau5, beta0);
-  beta1 = fdiv(beta1 + tau5, beta1);
-  beta2 = fdiv(beta2 + tau5, beta2);
+  beta0 = fdiv_normal(beta0 + tau5, beta0);
+  beta1 = fdiv_normal(beta1 + tau5, beta1);
+  beta2 = fdiv_normal(beta2 + tau5, beta2);
 
   double w0 = g0 * beta0 + eps, w1 = g1 * beta1 + eps, w2 = g2 * beta2 + eps;
-  double wsum = frcp(w0 + w1 + w2);
+  double wsum = fdiv_normal(1.0, w0 + w1 + w2);
   double l = w0 * (c00 * q0 + c01 * q1 + c02 * q2);
   l += w1 * (c10 * q1 + c11 * q2 + c12 * q3);
   l += w2 * (c20 * q2 + c21 * q3 + c22 * q4);
@@ -242,7 +289,7 @@ __device__ __forceinline__ void recon_weno5z(double q0, double q1, double q2, do
   w0 = g0 * beta2 + eps;
   w1 = g1 * beta1 + eps;
   w2 = g2 * beta0 + eps;
-  wsum = frcp(w0 + w1 + w2);
+  wsum = fdiv_normal(1.0, w0 + w1 + w2);
   double r = w0 * (c00 * q4 + c01 * q3 + c02 * q2);
   r += w1 * (c10 * q3 + c11 * q2 + c12 * q1);
   r += w2 * (c20 * q2 + c21 * q1 + c22 * q0);
@@ -251,7 +298,7 @@ __device__ __forceinline__ void recon_weno5z(double q0, double q1, double q2, do
 
   double dq = q3 - q2;
   dq = mc_limiter(q2 - q1, dq, 2.0);
-  const double alin = fdiv(2.0 * al * ar, al + ar);
+  const double alin = fdiv_normal(2.0 * al * ar, al + ar);
   ql = alin * l + (1.0 - alin) * (q2 + 0.5 * dq);
   qr = alin * r + (1.0 - alin) * (q2 - 0.5 * dq);
 }
@@ -264,7 +311,7 @@ __device__ __forceinline__ double mp5_edge(double fm2, double fm1, double f0, do
                                            double fp2) {
   constexpr double alpha = 4.0, epsm = 1.e-12;
   double f = 2.0 * fm2 - 13.0 * fm1 + 47.0 * f0 + 27.0 * fp1 - 3.0 * fp2;
-  f = kFluxFast ? f * (1.0 / 60.0) : f / 60.0;
+  f = kFluxFast ? f * (1.0 / 60.0) : ddiv(f, 60.0);
   const double fmp = f0 + minmod2(fp1 - f0, alpha * (f0 - fm1));
   if ((f - f0) * (f - fmp) <= epsm) return f;
   const double d2m = fm2 + f0 - 2.0 * fm1;
@@ -348,7 +395,7 @@ struct SphericalKSMetric {  // spherical_kerr_schild.hpp:42-243, X = (r, theta, 
     const double a2 = a * a;
     const double r = fabs(X1), cth = cos(X2), sth = sin(X2);
     const double sth2 = sth * sth, rho2 = r * r + a2 * cth * cth;
-    alpha_ = sqrt(ratio(rho2, 2 * r + rho2));
+    alpha_ = dsqrt(ratio(rho2, 2 * r + rho2));
     beta0_ = ratio(2 * r, 2 * r + rho2);
     g01_ = ratio(2 * r, rho2);
     g00_ = -1 + g01_;
@@ -361,8 +408,8 @@ struct SphericalKSMetric {  // spherical_kerr_schild.hpp:42-243, X = (r, theta, 
     c02_ = ratio(a, rho2);
     c11_ = ratio(1, rho2);
     c22_ = ratio(1, rho2 * sth2);
-    detgamma_ = sqrt(fabs(rho2 * (2 * r + rho2) * sth2));
-    detg_ = sqrt(fabs(rho2 * rho2 * sth2));
+    detgamma_ = dsqrt(fabs(rho2 * (2 * r + rho2) * sth2));
+    detg_ = dsqrt(fabs(rho2 * rho2 * sth2));
   }
   __device__ double alpha() const { return alpha_; }
   __device__ double beta(int i) const { return i == 0 ? beta0_ : 0.0; }
@@ -574,7 +621,7 @@ __device__ __forceinline__ Floors floors_at(const DevBounds &b, double x1, doubl
 }
 __device__ __forceinline__ double sie_floor_of(const DevBounds &b, const Floors &f, double rho) {
   return b.floor_type == PHX_FLOOR_EXPX1_RHO_U
-             ? smax(f.sie / smax(rho, f.den), b.sie_min_eos)
+             ? smax(ddiv(f.sie, smax(rho, f.den)), b.sie_min_eos)
              : f.sie;
 }
 
@@ -583,7 +630,7 @@ __device__ __forceinline__ double eos_p_rho_sie(const DevParams &p, double rho, 
   return p.gm1 * rho * sie;
 }
 __device__ __forceinline__ double eos_t_rho_sie(const DevParams &p, double sie) {
-  return sie / p.cv;
+  return ddiv(sie, p.cv);
 }
 __device__ __forceinline__ double eos_p_rho_t(const DevParams &p, double rho, double t) {
   return p.gm1 * rho * p.cv * t;
@@ -625,8 +672,8 @@ __device__ __forceinline__ void prim_to_flux(const DevParams &p, const int dir, 
   double vcon[3] = {fdiv(vpcon[0], W), fdiv(vpcon[1], W), fdiv(vpcon[2], W)};
   const double vel = vcon[dir];
   double Bcon[3] = {0.0, 0.0, 0.0};
-  const double u = (q[4] / rho > sie_floor ? (q[4] / rho > sie_max ? rho * sie_max : q[4])
-                                            : rho * sie_floor);
+  const double sie = ddiv(q[4], rho);
+  const double u = (sie > sie_floor ? (sie > sie_max ? rho * sie_max : q[4]) : rho * sie_floor);
   const double P = smax(q[L::prs], 0.0);
   const double gamma1 = q[L::gm1];
   if constexpr (MHD) {
@@ -646,9 +693,8 @@ __device__ __forceinline__ void prim_to_flux(const DevParams &p, const int dir, 
         BdotB += g.gcov(m + 1, n + 1) * Bcon[m] * Bcon[n];
       }
     }
-  const double vsq_max = 1.0 - 1.0 / (gam_max * gam_max);
-  if (vsq > vsq_max) {
-    double scale = fdiv(vsq_max, vsq);
+  if (vsq > p.vsq_max) {
+    double scale = fdiv(p.vsq_max, vsq);
     vsq *= scale;
     scale = fsqrt(scale);
     Bdotv *= scale;
@@ -740,13 +786,13 @@ __device__ __forceinline__ void signal_speeds(double rho, double u, double pr, d
                                               const double v[3], double vsq, double gam1,
                                               const M &g, double sig[3]) {
   const double rho_rel = rho + u + pr;
-  const double vasq = bsq / (rho_rel + bsq);
-  double cssq = gam1 * pr / rho_rel;
+  const double vasq = ddiv(bsq, rho_rel + bsq);
+  double cssq = ddiv(gam1 * pr, rho_rel);
   cssq += vasq - cssq * vasq;
-  const double vcoff = g.alpha() / (1.0 - vsq * cssq);
+  const double vcoff = ddiv(g.alpha(), 1.0 - vsq * cssq);
 #pragma unroll
   for (int m = 0; m < 3; ++m) {
-    const double vpm = sqrt(cssq * (1.0 - vsq) *
+    const double vpm = dsqrt(cssq * (1.0 - vsq) *
                             (g.gcon(m, m) * (1.0 - vsq * cssq) - v[m] * v[m] * (1.0 - cssq)));
     const double bm = M::nz_beta(m) ? g.beta(m) : 0.0;
     const double vp = vcoff * (v[m] * (1.0 - cssq) + vpm) - bm;
@@ -766,8 +812,8 @@ __device__ __forceinline__ void p2c(const double rho, const double vp[3], const 
 #pragma unroll
     for (int jj = 0; jj < 3; ++jj)
       if (M::nz_cov(ii + 1, jj + 1)) vsq0 += g.gcov(ii + 1, jj + 1) * vp[ii] * vp[jj];
-  const double W = sqrt(1. + vsq0);
-  const double iW = 1.0 / W;
+  const double W = dsqrt(1. + vsq0);
+  const double iW = ddiv(1.0, W);
   const double v[3] = {vp[0] * iW, vp[1] * iW, vp[2] * iW};
 #pragma unroll
   for (int ii = 0; ii < 3; ++ii)
@@ -785,10 +831,10 @@ __device__ __forceinline__ void p2c(const double rho, const double vp[3], const 
   double bsq = 0.0;
   double bcov[3] = {0.0, 0.0, 0.0};
   if constexpr (MHD) {
-    bcon[0] = W * Bdotv / g.alpha();
+    bcon[0] = ddiv(W * Bdotv, g.alpha());
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
-      const double sh = M::nz_beta(m) ? g.beta(m) / g.alpha() : 0.0;
+      const double sh = M::nz_beta(m) ? ddiv(g.beta(m), g.alpha()) : 0.0;
       bcon[m + 1] = b[m] * iW + Bdotv * W * (v[m] - sh);
     }
     bsq = Bsq * iW * iW + Bdotv * Bdotv;
@@ -869,17 +915,17 @@ struct Residual {
     const double rbarsq = rbarsq_mu(mu, x);
     const double qbar = qbar_mu(mu, x);
     const double vhatsq = vhatsq_mu(mu, rbarsq);
-    const double iWhat = sqrt(1.0 - vhatsq);
+    const double iWhat = dsqrt(1.0 - vhatsq);
     const double What = ratio(1.0, iWhat);
     const double rhohat = rhohat_mu(iWhat);
     const double ehat = ehat_mu(mu, qbar, rbarsq, vhatsq, What);
     const double Phat = eos_p_rho_sie(*p, rhohat, ehat);
     const double hhat = rhohat * (1.0 + ehat) + Phat;
-    const double ahat = Phat / make_positive(hhat - Phat);
+    const double ahat = ddiv(Phat, make_positive(hhat - Phat));
     const double nua = (1.0 + ahat) * (1.0 + ehat) * iWhat;
     const double nub = (1.0 + ahat) * (1.0 + qbar - mu * rbarsq);
     const double nuhat = smax(nua, nub);
-    const double muhat = 1.0 / (nuhat + mu * rbarsq);
+    const double muhat = ddiv(1.0, nuhat + mu * rbarsq);
     return mu - muhat;
   }
 };
@@ -916,7 +962,7 @@ __device__ __forceinline__ bool regula_falsi(F &f, double a, double b, double to
   yb *= sign;
   int b1 = 0, b2 = 0;
   while (b - a > 2.0 * tol && it < max_iter) {
-    const double c = (a * yb - b * ya) / (yb - ya);
+    const double c = ddiv(a * yb - b * ya, yb - ya);
     if (c == a) {
       b = a;
       it++;
@@ -962,7 +1008,7 @@ __device__ __forceinline__ double regula_falsi_bracketed(F &f, double a, double 
   yb *= sign;
   int b1 = 0, b2 = 0;
   while (b - a > 2.0 * tol && it < max_iter) {
-    const double c = (a * yb - b * ya) / (yb - ya);
+    const double c = ddiv(a * yb - b * ya, yb - ya);
     if (c == a) {
       b = a;
       it++;
@@ -1010,10 +1056,9 @@ __device__ __forceinline__ bool c2p_setup(const DevParams &p, const M &g, const 
                                           const double *cons, double *prim,
                                           C2PState<MHD> &z) {
   if (isnan(cons[0]) + isnan(cons[1]) + isnan(cons[4]) > 0) return false;
-  const double igdet = 1.0 / g.detgamma();
+  const double igdet = ddiv(1.0, g.detgamma());
   Floors fl = floors_at(p.bnd, X[0], X[1], X[2]);
   const double rhoflr = fl.rho * p.fsf;
-  const double gam_max = p.bnd.gam_max;
   const double D = cons[0] * igdet;
   const double tau = cons[4] * igdet;
   const double q = ratio(tau, D);
@@ -1033,7 +1078,7 @@ __device__ __forceinline__ bool c2p_setup(const DevParams &p, const M &g, const 
   if constexpr (MHD) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) prim[5 + i] = cons[5 + i] * igdet;
-    const double sD = 1.0 / sqrt(smax(D, rhoflr));
+    const double sD = ddiv(1.0, dsqrt(smax(D, rhoflr)));
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       z.bu[i] = prim[5 + i] * sD;
@@ -1050,7 +1095,7 @@ __device__ __forceinline__ bool c2p_setup(const DevParams &p, const M &g, const 
   }
   z.bdotr = bdotr;
   const double zsq = rsq / 1.0;
-  const double v0sq = smin(zsq / (1.0 + zsq), 1.0 - 1.0 / (gam_max * gam_max));
+  const double v0sq = smin(ddiv(zsq, 1.0 + zsq), p.vsq_max);
   Residual<MHD> &res = z.res;
   res.p = &p;
   res.D = D; res.q = q; res.bsq = bsq; res.bsq_rpsq = bsq_rpsq; res.rsq = rsq;
@@ -1073,15 +1118,15 @@ __device__ __forceinline__ double c2p_unwrap(const DevParams &p, const M &g, C2P
   const double x = res.x_mu(mu);
   const double rbarsq = res.rbarsq_mu(mu, x);
   const double vsq = res.vhatsq_mu(mu, rbarsq);
-  const double iW = sqrt(1.0 - vsq);
+  const double iW = dsqrt(1.0 - vsq);
   prim[0] = res.rhohat_mu(iW);
   const double qbar = res.qbar_mu(mu, x);
-  const double W = 1.0 / iW;
+  const double W = ddiv(1.0, iW);
   prim[4] = res.ehat_mu(mu, qbar, rbarsq, vsq, W);
   temp = eos_t_rho_sie(p, prim[4]);
   prim[4] *= prim[0];
   prim[L::prs] = eos_p_rho_t(p, prim[0], temp);
-  prim[L::gm1] = eos_bmod_rho_t(p, prim[0], temp) / prim[L::prs];
+  prim[L::gm1] = ddiv(eos_bmod_rho_t(p, prim[0], temp), prim[L::prs]);
   double vel[3], bu[3] = {z.bu[0], z.bu[1], z.bu[2]};
 #pragma unroll
   for (int i = 0; i < 3; ++i) {

@@ -315,9 +315,9 @@ __device__ __forceinline__ double cell_dt(const BlockGeom &bg, const PackEntry &
   for (int d = 0; d < 3; ++d) {
     if (d >= bg.ndim) break;
     const double s = smax(E.csig[d * n + c], smax(E.fsig[d * n + c], E.fsig[d * n + c + off[d]]));
-    ldt += s / bg.dx[d];
+    ldt += ddiv(s, bg.dx[d]);
   }
-  const double t = 1.0 / (ldt + 1.e-50);
+  const double t = ddiv(1.0, ldt + 1.e-50);
   return isnan(t) ? DBL_MAX : t;  // a NaN time constrains nothing (as a serial minimum)
 }
 

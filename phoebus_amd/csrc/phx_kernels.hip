@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void k_update(BlockGeom b, FluxPtrs flux, Cons
       const double *F3 = flux[16 + l];
       du += a3 * F3[c + (long)b.ni * b.nj] - a3 * F3[c];
     }
-    double dudt = -du / vol;
+    double dudt = ddiv(-du, vol);
     if (src[l] != nullptr && l >= 1 && l <= 4) dudt = dudt + src[l][c];
     const double us = beta * u_stage[l][c] + (1 - beta) * u_base[l][c];
     u_stage[l][c] = us;
@@ -192,9 +192,9 @@ __global__ __launch_bounds__(256) void k_dt_partial(BlockGeom b, const double *_
         const long off = d == 0 ? 1 : d == 1 ? (long)b.ni : (long)b.ni * b.nj;
         s = smax(s, smax(fsig[d * n + c], fsig[d * n + c + off]));
       }
-      ldt += s / b.dx[d];
+      ldt += ddiv(s, b.dx[d]);
     }
-    lmin = smin(lmin, 1.0 / (ldt + 1.e-50));
+    lmin = smin(lmin, ddiv(1.0, ldt + 1.e-50));
   }
   lmin = block_min(lmin);
   if (threadIdx.x == 0) partial[blockIdx.x] = lmin;
@@ -610,6 +610,7 @@ DevParams make_dev_params(const phx_fluid_params *p) {
   d.bnd.sie_min_eos = p->bounds.sie_min_eos;
   d.bnd.gam_max = p->bounds.gam_max;
   d.bnd.sie_max = p->bounds.sie_max;
+  d.vsq_max = 1.0 - 1.0 / (p->bounds.gam_max * p->bounds.gam_max);
   const phx_mgr &m = p->geom.mgr;
   d.mgr.derefine_poles = m.derefine_poles;
   d.mgr.h = m.h;

@@ -121,7 +121,7 @@ __device__ __forceinline__ double update_con2prim_body(
       double du = a1 * f[0][1] - a1 * f[0][0];
       if constexpr (NDIM >= 2) du += a2 * f[1][1] - a2 * f[1][0];
       if constexpr (NDIM == 3) du += a3 * f[2][1] - a3 * f[2][0];
-      double dudt = -du / vol;
+      double dudt = ddiv(-du, vol);
       if constexpr (SRC) {
         if (l >= 1 && l <= 4) dudt = dudt + src[l][c];
       }
@@ -169,12 +169,12 @@ __device__ __forceinline__ double update_con2prim_body(
         if (d >= b.ndim) break;
         const long off = d == 0 ? 1 : d == 1 ? sj : sk;
         const double s = smax(sig[d], smax(fsig[d * n + c], fsig[d * n + c + off]));
-        ldt += s / b.dx[d];
+        ldt += ddiv(s, b.dx[d]);
       }
       // a NaN time (a zone whose speeds are NaN, e.g. P = 0 on the energy floor, where
       // Gamma_1 = 0/0 as in the reference) constrains nothing: the serial minimum of the
       // reference and of k_dt_partial never lets a NaN replace a number
-      const double t = 1.0 / (ldt + 1.e-50);
+      const double t = ddiv(1.0, ldt + 1.e-50);
       ldt_min = isnan(t) ? DBL_MAX : t;
     }
   }

@@ -210,6 +210,60 @@ def test_batch_floor_profiles(phx, ftype, mhd):
     assert np.all(np.abs(out[:5] - ref["cons"][:5]) <= 1e-7 * cscale)
 
 
+@pytest.mark.parametrize("mhd", [False, True])
+@pytest.mark.parametrize("scale", [1e-60, 1e-30, 1.0, 1e30, 1e60])
+def test_division_range_bits(phx, scale, mhd):
+    """The library's division and square root round as IEEE over the magnitudes the fluid
+    path can meet: batched p2c and con2prim, and the fluxes of a block that is uniform on
+    one side of a jump (the WENO weights then span 1e100 and more), equal the oracle's bits
+    for states scaled by 1e-60 .. 1e60."""
+    say(f"[gpu] division range scale={scale} mhd={mhd}")
+    gamma, n = 13.0 / 9.0, 1023
+    rng = np.random.default_rng(77)
+
+    def scaled(pr):
+        pr = pr.copy()
+        pr[0] *= scale
+        pr[4] *= scale
+        pr[-2] *= scale
+        if mhd:
+            pr[5:8] *= np.sqrt(scale)
+        return np.ascontiguousarray(pr)
+
+    p = fluid_params(gamma=gamma, mhd=mhd, c2p_tol=1e-10)
+    op = oparams(p)
+    prims, coords = scaled(PH.random_prims(rng, n, mhd, gamma, wmax=5.0)), np.zeros((2, n))
+    cons = O.p2c_batch(op, coords, prims)
+    ref = O.c2p_batch(op, coords, cons)
+    d_prim, d_cons = DeviceArray.from_host(prims), DeviceArray(cons.shape)
+    phx.prim_to_con_batch(p, n, None, d_prim, d_cons)
+    synchronize()
+    assert np.array_equal(d_cons.get(), cons)
+    d_mu, d_fail = DeviceArray.from_host(np.zeros(n)), DeviceArray((n,))
+    phx.con2prim_batch(p, n, None, d_cons, d_prim, d_mu, d_fail)
+    synchronize()
+    assert np.array_equal(d_fail.get(), ref["fail"])
+    assert np.array_equal(d_mu.get(), ref["mu"], equal_nan=True)
+    assert np.array_equal(d_prim.get(), ref["prim"], equal_nan=True)
+    for recon in (A.RECON_WENO5Z, A.RECON_MP5):
+        b = geom_block(3, (10, 9, 8), A.GEOM_MINKOWSKI)
+        q = fluid_params(gamma=gamma, mhd=mhd, recon=recon, riemann=A.RIEMANN_HLL)
+        prim = random_block(rng, b, mhd, gamma, A.GEOM_MINKOWSKI)
+        prim[..., :9] = prim[..., :1, :1, :1]  # uniform for i < 9, random beyond
+        prim = scaled(prim)
+        rf, rs = O.calculate_fluxes(oparams(q), oblock(b), prim)
+        st = BlockState(q, b)
+        st.prim.upload(prim)
+        phx.calculate_fluxes(q, b, st.fields())
+        synchronize()
+        gf, gs = st.flux.get(), st.face_sig.get()
+        for d in range(3):
+            sl = consumed_face_slices(b, d)
+            assert np.array_equal(gs[d][sl], rs[d][sl], equal_nan=True), (recon, d)
+            for m in range(rf.shape[1]):
+                assert np.array_equal(gf[d, m][sl], rf[d, m][sl], equal_nan=True), (recon, d, m)
+
+
 def test_batch_edge_sizes(phx):
     # an empty batch is a no-op (no pointer is read), a negative one is refused, and ragged
     # sizes (not multiples of a wave or a 256-lane group) match the oracle bit for bit and
