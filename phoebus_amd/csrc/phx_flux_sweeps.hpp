@@ -76,7 +76,7 @@ __device__ __forceinline__ void flux_x_body(const DevParams &p, const BlockGeom 
     double q[2 * H + 1];
 #pragma unroll
     for (int o = 0; o < 2 * H + 1; ++o) q[o] = stage[v][recon_ok ? t + o - H : t];
-    reconstruct_edges<RECON>(q, up[v], lo[v]);
+    reconstruct_edges<RECON, GEOM != PHX_GEOM_MINKOWSKI>(q, up[v], lo[v]);
     pin(up[v]);
     pin(lo[v]);
   }
@@ -147,7 +147,7 @@ __device__ __forceinline__ void flux_tile_body(const DevParams &p, const BlockGe
 #pragma unroll
     for (int oo = 0; oo < 2 * H + 1; ++oo)
       q[oo] = live ? lds[v * plane + (recon_ok ? me + (oo - H) * ti_n : me)] : 0.0;
-    reconstruct_edges<RECON>(q, up[v], lo[v]);
+    reconstruct_edges<RECON, GEOM != PHX_GEOM_MINKOWSKI>(q, up[v], lo[v]);
     pin(up[v]);
     pin(lo[v]);
   }
@@ -248,7 +248,7 @@ __device__ __forceinline__ void flux_march_body(const DevParams &p, const BlockG
       double q[2 * H + 1];
 #pragma unroll
       for (int o = 0; o < 2 * H + 1; ++o) q[o] = ring[(v * Q + sl[o]) * ti + cl];
-      reconstruct_edges<RECON>(q, up[v], lo[v]);
+      reconstruct_edges<RECON, GEOM != PHX_GEOM_MINKOWSKI>(q, up[v], lo[v]);
       pin(up[v]);
       pin(lo[v]);
     }
