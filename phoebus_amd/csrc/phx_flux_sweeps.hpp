@@ -321,9 +321,15 @@ __global__ __launch_bounds__(512) void k_pack_flux_tile(DevParams p, PackView v,
       contig(E.flux, E.bg.ncell), E.fsig, lds);
 }
 
+// waves per SIMD the marching kernels over packs are built for: four (128 VGPRs) on Minkowski
+// and, in the fast arithmetic, on FMKS with its cached metric (139-143 VGPRs and three waves
+// if left alone, 3-4 registers spilled at four: 5 % of the pack's RK2 step)
+constexpr int march_waves(int geom) {
+  return geom == PHX_GEOM_MINKOWSKI || (kFluxFast && geom == PHX_GEOM_FMKS) ? 4 : 1;
+}
 template <int DIR, int RECON, int RIEMANN, int GEOM, int TI>
 __global__ __launch_bounds__(kMarchLanes)
-__attribute__((amdgpu_waves_per_eu(GEOM == PHX_GEOM_MINKOWSKI ? 4 : 1))) void k_pack_flux_march(DevParams p, PackView v, int ti,
+__attribute__((amdgpu_waves_per_eu(march_waves(GEOM)))) void k_pack_flux_march(DevParams p, PackView v, int ti,
                                                                  int nseg) {
   extern __shared__ double lds[];
   const long g = xcd_remap(blockIdx.x, gridDim.x);

@@ -71,6 +71,35 @@ def test_fast_fluxes_match_oracle(phx, case):
     say(f"    largest difference {worst:.2e} of the component scale")
 
 
+@pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
+@pytest.mark.parametrize("mhd", [False, True])
+def test_fast_curved_fluxes_at_the_bounds(phx, geom, mhd):
+    """The curved-metric face states with every bound acting on a share of the faces (density
+    and energy floors, Lorentz-factor and energy ceilings), next to a uniform half whose
+    smoothness indicators vanish, at the block test's tolerance."""
+    say(f"[gpu] fast curved fluxes at the bounds, geom {geom} mhd {mhd}")
+    rng = np.random.default_rng(90 + geom)
+    b = geom_block(3, (13, 10, 9), geom)
+    prim = random_block(rng, b, mhd, 13.0 / 9.0, geom)
+    prim[..., :9] = prim[..., :1, :1, :1]
+    for recon, riemann in ((A.RECON_WENO5Z, A.RIEMANN_HLL), (A.RECON_LINEAR, A.RIEMANN_LLF)):
+        p = geom_params(geom, gamma=13.0 / 9.0, mhd=mhd, recon=recon, riemann=riemann,
+                        floors=dict(rho0=float(np.median(prim[0])), sie0=0.5),
+                        ceilings=(1.5, 1.0))
+        p.flux_arith = A.FLUX_ARITH_FAST
+        rf, rs = O.calculate_fluxes(oparams(p), oblock(b), prim)
+        st = BlockState(p, b)
+        st.prim.upload(prim)
+        phx.calculate_fluxes(p, b, st.fields())
+        synchronize()
+        gf, gs = st.flux.get(), st.face_sig.get()
+        for d in range(3):
+            sl = consumed_face_slices(b, d)
+            for m in range(rf.shape[1]):
+                _flux_close(gf[d, m][sl], rf[d, m][sl], f"recon={recon} d={d} m={m}")
+            _flux_close(gs[d][sl], rs[d][sl], f"face_sig d={d}")
+
+
 def test_fast_sweep_shapes_agree(phx):
     say("[gpu] fast flux arithmetic: every y/z sweep shape, bit for bit")
     rng = np.random.default_rng(91)
