@@ -290,9 +290,9 @@ int phx_prim_to_con_batch(phx_ctx *ctx, const phx_fluid_params *p, int64_t n,
  * the sweep; with ts < 0, one 64-lane wave of ti columns (a power of two) by 64 / ti rows
  * marching along the sweep in -ts segments of the faces.  Results do not depend on the
  * shape.  reps = timed launches per candidate.  phx_tile_shape reports the shape in use
- * for dir 1 (y) or 2 (z); phx_set_tile_shape fixes one (ts = 0: the default, marching
- * waves of 8 x 8 in segments of at least 24 faces where that makes >= 1024 waves, else
- * tiles of 8 x up to 64). */
+ * for dir 1 (y) or 2 (z); phx_set_tile_shape fixes one (ts = 0: the default, marching waves
+ * of 8 x 8 or tiles of 8 x 32, whichever takes fewer wave-steps on the block; tiles for
+ * the constant and linear reconstructions). */
 int phx_autotune(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
                  const phx_block_fields *f, int reps, phx_stream stream);
 int phx_tile_shape(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b, int dir,

@@ -35,15 +35,36 @@ TileShape resolve_tile_shape(int d, int recon, int mhd, const BlockGeom &bg, Til
   const int H = recon == PHX_RECON_CONSTANT ? 0 : recon == PHX_RECON_LINEAR ? 1 : 2;
   const int NP = mhd ? 10 : 7;
   if (want.ts == 0) {
-    // the default: marching waves of 8 columns x 8 rows in segments of at least 24 faces
-    // when that fills the chip with at least 1024 waves; a small block's march would be a
-    // few waves stepping serially, so it keeps 8-wide tiles of up to 64 rows
+    // The default.  The sweeps are bound by VALU issue, so the shape with the fewest
+    // wave-steps (one 64-lane reconstruction and flux) wins once there are enough waves: a
+    // marching wave's first row of a segment only starts it, a tile's 2H + 1 edge rows are
+    // redone by its neighbours.  A wave-step of a tile is cheaper (no ring, no barriers
+    // between steps): 7.0 against 8.8 ns per SIMD at 64^3, 6.3 against 7.0 at 96^3 (exact
+    // arithmetic), hence the 0.83.  Marching segments of about three steps where that still
+    // makes four waves per SIMD (4096), else single-step segments for the most waves.
+    // Tiles of 8 x 32: 27 faces per 32 rows, 4 waves and 20 KB each, so eight per CU.
+    // Measured (us, exact arithmetic, y sweep; the choice first): 128^3 fast 8 x -6 176
+    // against 193; 96^3 8 x -5 116 / 125; 64^3 8 x -10 47 / 49; 48^3 8 x 32 26.0 / 28.3;
+    // 32^3 8 x -5 15.7 / 19.7; 100 x 75 x 51 8 x 32 61 / 59.  (Segments of at least 24 faces
+    // from 1024 waves on, tiles of up to 64 rows below, took 189, 143, 75, 34, 20 and 79.)
+    // Without the 5-point stencils a wave-step is too short to pay for the ring: tiles.
+    const int ti = want.ti > 0 ? want.ti : 8;
+    const TileShape t = resolve_tile_shape(d, recon, mhd, bg, TileShape{ti, 32});
+    if (H < 2) return t;
     const int nf = bg.ie[d] - bg.is[d] + 3;
-    const int nseg = nf / 24 < 1 ? 1 : nf / 24 > 8 ? 8 : nf / 24;
-    const TileShape m =
-        resolve_tile_shape(d, recon, mhd, bg, TileShape{want.ti > 0 ? want.ti : 8, -nseg});
-    if (flux_march_groups(bg, d, m.ti, -m.ts) >= 1024) return m;
-    want.ts = 64;
+    TileShape m = resolve_tile_shape(d, recon, mhd, bg, TileShape{ti, -1});
+    const int MR = kMarchLanes / m.ti;
+    auto steps = [&](int nseg) { return (nf + nseg + MR - 1) / MR; };  // of a column
+    const long chunks = flux_march_groups(bg, d, m.ti, 1);
+    int nseg = (steps(1) + 2) / 3;
+    nseg = (steps(nseg) + 2) / 3;
+    if (chunks * nseg < 4096) nseg = MR > 1 ? (nf + MR - 2) / (MR - 1) : nf;
+    m = resolve_tile_shape(d, recon, mhd, bg, TileShape{m.ti, -nseg});
+    const long tile_steps = flux_tile_groups(bg, d, t.ti, t.ts, H) * ((t.ti * t.ts + 63) / 64);
+    // (under half a wave per SIMD both are one launch's latency, and the tiles' is shorter: 16^3
+    // 12.9 against 13.5, 24^3 13.8 / 14.0)
+    const long march_steps = chunks * steps(-m.ts);
+    return march_steps >= 512 && (double)march_steps < 0.83 * (double)tile_steps ? m : t;
   }
   if (want.ts < 0) {  // marching: ti a power of two up to 64, -ts segments of the faces
     const int want_ti = want.ti > 0 ? want.ti : 8;

@@ -175,8 +175,13 @@ __device__ __forceinline__ void flux_tile_body(const DevParams &p, const BlockGe
 // the column count ti is that constant (the launchers pass it for the common widths), so
 // the ring's row and variable strides fold into the LDS instructions' offsets instead of
 // run-time multiplies; TI = 0: ti as passed
+// SEG_FIRST: the segments of a column are consecutive workgroups.  Each XCD takes a contiguous
+// range of groups (xcd_remap), and the first segments may march one step more than the last, so
+// over one block with the columns fastest whole XCDs drew long or short waves only (96^3 in 5
+// segments 124 -> 116 us, 100 x 75 x 51 in 3 69 -> 56).  A pack's XCDs take several blocks each;
+// there the columns go fastest, whose neighbours share cache lines (1.4 % of the RK2 step).
 template <int DIR, int RECON, int RIEMANN, bool MHD, int GEOM, bool CACHED = false, int TI = 0,
-          class PP, class FP>
+          bool SEG_FIRST = false, class PP, class FP>
 __device__ __forceinline__ void flux_march_body(const DevParams &p, const BlockGeom &b, long bx,
                                                 int ti_run, int nseg, const PP &prim,
                                                 const FP &flux,
@@ -191,8 +196,8 @@ __device__ __forceinline__ void flux_march_body(const DevParams &p, const BlockG
   const int nci = b.ie[0] - b.is[0] + 3;  // i over [is-1, ie+1]
   const long ncol = (long)nci * (b.ie[T] - b.is[T] + 1 + 2 * dt_);
   const long nchunk = (ncol + ti - 1) / ti;
-  const int sg = (int)(bx / nchunk);
-  long col = (bx % nchunk) * ti + (lane & (ti - 1));
+  const int sg = (int)(SEG_FIRST ? bx % nseg : bx / nchunk);
+  long col = (SEG_FIRST ? bx / nseg : bx % nchunk) * ti + (lane & (ti - 1));
   const bool colv = col < ncol;
   if (!colv) col = ncol - 1;
   const int i = b.is[0] - 1 + (int)(col % nci);
@@ -284,7 +289,7 @@ __attribute__((amdgpu_waves_per_eu(GEOM == PHX_GEOM_MINKOWSKI ? 4 : 1))) void k_
                                                             FluxPtrs flux,
                                                             double *__restrict__ fsig) {
   extern __shared__ double lds[];
-  flux_march_body<DIR, RECON, RIEMANN, MHD, GEOM, false, TI>(
+  flux_march_body<DIR, RECON, RIEMANN, MHD, GEOM, false, TI, true>(
       p, b, xcd_remap(blockIdx.x, gridDim.x), ti, nseg, prim, flux, fsig, lds);
 }
 

@@ -30,6 +30,22 @@ TileShape pack_shape(const phx_pack *k, int d, TileShape want) {
   return best;
 }
 
+// the shape a pack starts with: its blocks share the launch, so the march needs fewer segments
+// than each block's own default would take: the fewest that make two rounds of four waves per
+// SIMD over the pack, up to 8 (40 FMKS torus blocks, y / z sweep: 8 x -1, 6120 waves, 300 /
+// 301 us; 8 x -2 258 / 253); tiles where the stencil is short, as for single blocks
+static TileShape pack_default_shape(const phx_pack *k, int d) {
+  if (k->p.recon < PHX_RECON_WENO5Z) return pack_shape(k, d, TileShape{8, 32});
+  TileShape t;
+  for (int nseg = 1; nseg <= 8; ++nseg) {
+    t = pack_shape(k, d, TileShape{8, -nseg});
+    long waves = 0;
+    for (const auto &g : k->geoms) waves += pack_groups_flux(d, k->p.recon, g, t);
+    if (waves >= 8192) break;
+  }
+  return t;
+}
+
 int build_start(phx_pack *k, int kind) {
   std::vector<long> st(k->n + 1, 0);
   for (int b = 0; b < k->n; ++b) {
@@ -205,7 +221,7 @@ int phx_pack_create(phx_ctx *ctx, const phx_fluid_params *p, int nblocks,
       e[st - 1].push_back(x);
     }
   }
-  for (int d = 0; d < 3; ++d) k->tiles[d] = pack_shape(k, d, TileShape());
+  for (int d = 0; d < 3; ++d) k->tiles[d] = d == 0 ? TileShape() : pack_default_shape(k, d);
   bool ok = true;
   for (int st = 0; st < 2 && ok; ++st)
     ok = hipMalloc(&k->entries[st], sizeof(PackEntry) * nblocks) == hipSuccess &&
