@@ -292,7 +292,9 @@ int phx_prim_to_con_batch(phx_ctx *ctx, const phx_fluid_params *p, int64_t n,
  * shape.  reps = timed launches per candidate.  phx_tile_shape reports the shape in use
  * for dir 1 (y) or 2 (z); phx_set_tile_shape fixes one (ts = 0: the default, marching waves
  * of 8 x 8 or tiles of 8 x 32, whichever takes fewer wave-steps on the block; tiles for
- * the constant and linear reconstructions). */
+ * the constant and linear reconstructions).  While a block's shapes are the defaults, the
+ * sweeps of all directions go in one launch where that is faster (small blocks, and any
+ * block with the constant and linear reconstructions); phx_autotune times that too. */
 int phx_autotune(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
                  const phx_block_fields *f, int reps, phx_stream stream);
 int phx_tile_shape(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b, int dir,

@@ -91,6 +91,36 @@ TileShape resolve_tile_shape(int d, int recon, int mhd, const BlockGeom &bg, Til
   return t;
 }
 
+// every direction's groups for one launch of 256-lane groups: x rows and tiles of up to 8 x 32,
+// each direction starting at a multiple of 8 groups
+FluxGroups all_flux_groups(int recon, int mhd, const BlockGeom &bg) {
+  const int H = recon == PHX_RECON_CONSTANT ? 0 : recon == PHX_RECON_LINEAR ? 1 : 2;
+  FluxGroups fg{};
+  fg.n[0] = (unsigned)flux_x_groups(bg, H);
+  for (int d = 1; d < 3; ++d) {
+    fg.off[d] = (fg.off[d - 1] + fg.n[d - 1] + 7) / 8 * 8;
+    if (d >= bg.ndim) continue;
+    const TileShape t = resolve_tile_shape(d, recon, mhd, bg, TileShape{8, 32});
+    fg.n[d] = (unsigned)flux_tile_groups(bg, d, t.ti, t.ts, H);
+    fg.ti[d] = t.ti;
+    fg.ts[d] = t.ts;
+  }
+  fg.off[3] = fg.off[2] + fg.n[2];
+  return fg;
+}
+
+// One launch in place of two or three: a small block's sweeps are each one launch's latency on
+// a part of the chip (16^3: 13 us apiece on 41-54 of 256 CUs), and on larger blocks each
+// launch ends in a partial round.  Whole stage, one launch against separate ones in their
+// default shapes (us): 16^3 36.5 / 57.3, 32^3 57.2 / 62.7, 48^3 92 / 109, 64^3 171 / 180,
+// 100 x 75 x 51 (5,824 groups) 216 / 239, 2-D 256 x 128 42 / 48; 96^3 (14,171) fast 412 / 400: from
+// about 8,192 groups on, the 5-point stencils' marching waves win.  The shorter stencils
+// sweep in tiles on any block (150 x 90 x 70 hydro PLM 201 / 218).
+bool one_launch_fluxes(int recon, int mhd, const BlockGeom &bg) {
+  if (bg.ndim == 1) return false;
+  return recon < PHX_RECON_WENO5Z || all_flux_groups(recon, mhd, bg).off[3] <= 8192;
+}
+
 long pack_groups_flux(int d, int recon, const BlockGeom &bg, TileShape shape) {
   const int H = recon == PHX_RECON_CONSTANT ? 0 : recon == PHX_RECON_LINEAR ? 1 : 2;
   if (d == 0) return flux_x_groups(bg, H);

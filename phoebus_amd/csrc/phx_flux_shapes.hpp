@@ -50,6 +50,13 @@ __host__ __device__ inline long flux_tile_groups(const BlockGeom &b, int dir, in
   return nic * nft * ntr;
 }
 
+// a launch of k_flux_tile: direction d takes groups [off[d], off[d] + n[d]), off[3] in all
+constexpr int kAllDirs = 3;  // launch_fluxes' direction for the three sweeps in one launch
+struct FluxGroups {
+  unsigned n[3], off[4];
+  int ti[3], ts[3];
+};
+
 // ---- y, z marching: one wave per workgroup --------------------------------------------
 // A wave holds ti columns (consecutive in the flattened face range of (i, transverse
 // index), i fastest) by MR = 64 / ti rows along the sweep, and marches over one of nseg

@@ -293,13 +293,28 @@ __attribute__((amdgpu_waves_per_eu(GEOM == PHX_GEOM_MINKOWSKI ? 4 : 1))) void k_
       p, b, xcd_remap(blockIdx.x, gridDim.x), ti, nseg, prim, flux, fsig, lds);
 }
 
-template <int DIR, int RECON, int RIEMANN, bool MHD, int GEOM>
-__global__ __launch_bounds__(512) void k_flux_tile(DevParams p, BlockGeom b, int ti_n,
-                                                    int ts_n, PrimPtrs prim, FluxPtrs flux,
+// the y and z sweeps in tiles, and on small blocks the x sweep with them in one launch
+// (fg: which directions, their groups and tile shapes; one_launch_fluxes).  Dynamic LDS
+// [NP][ts_n][ti_n] (primitives, then upper edges), or [NP][XB] for an x group.
+template <int RECON, int RIEMANN, bool MHD, int GEOM>
+__global__ __launch_bounds__(512) void k_flux_tile(DevParams p, BlockGeom b, FluxGroups fg,
+                                                    PrimPtrs prim, FluxPtrs flux,
                                                     double *__restrict__ fsig) {
-  extern __shared__ double lds[];  // [NP][ts_n][ti_n]: primitives, then upper edges
-  flux_tile_body<DIR, RECON, RIEMANN, MHD, GEOM>(p, b, (int)xcd_remap(blockIdx.x, gridDim.x),
-                                                 ti_n, ts_n, prim, flux, fsig, lds);
+  extern __shared__ double lds[];
+  // each direction's groups start at a multiple of 8, so their renumbering by XCD holds
+  const int d = blockIdx.x < fg.off[1] ? 0 : blockIdx.x < fg.off[2] ? 1 : 2;
+  const unsigned local = blockIdx.x - fg.off[d];
+  if (local >= fg.n[d]) return;
+  const int g = (int)xcd_remap(local, fg.n[d]);
+  if (d == 0)
+    flux_x_body<RECON, RIEMANN, MHD, GEOM>(p, b, g, prim, flux, fsig,
+                                           reinterpret_cast<double(*)[XB]>(lds));
+  else if (d == 1)
+    flux_tile_body<1, RECON, RIEMANN, MHD, GEOM>(p, b, g, fg.ti[1], fg.ts[1], prim, flux, fsig,
+                                                 lds);
+  else
+    flux_tile_body<2, RECON, RIEMANN, MHD, GEOM>(p, b, g, fg.ti[2], fg.ts[2], prim, flux, fsig,
+                                                 lds);
 }
 
 // ---- packs: the same sweeps over a work list of blocks --------------------------------
@@ -362,21 +377,21 @@ static void with_march_width(int ti, F &&f) {
 template <int RECON, int RIEMANN, bool MHD, int GEOM>
 static void launch_dir(int d, const DevParams &dp, const BlockGeom &bg, const PrimPtrs &prim,
                        const FluxPtrs &flux, double *fsig, hipStream_t s, TileShape shape) {
-  const int dj = bg.ndim > 1, dk = bg.ndim > 2;
   if (d == 0) {
-    constexpr int H = ReconWidth<RECON>::H;
-    const long total = (long)bg.ni * (bg.ie[1] - bg.is[1] + 1 + 2 * dj) *
-                       (bg.ie[2] - bg.is[2] + 1 + 2 * dk);
-    const long stride = XB - 2 * H - 1;
-    const unsigned blocks = (unsigned)((total - 2 * H - 1 + stride - 1) / stride);
+    const unsigned blocks = (unsigned)flux_x_groups(bg, ReconWidth<RECON>::H);
     hipLaunchKernelGGL((k_flux_x<RECON, RIEMANN, MHD, GEOM>), dim3(blocks), dim3(XB), 0, s, dp,
                        bg, prim, flux, fsig);
     return;
   }
+  if (d == kAllDirs) {
+    const FluxGroups fg = all_flux_groups(RECON, MHD, bg);
+    const size_t lds = sizeof(double) * (size_t)Layout<MHD>::nprim * XB;
+    hipLaunchKernelGGL((k_flux_tile<RECON, RIEMANN, MHD, GEOM>), dim3(fg.off[3]), dim3(XB), lds,
+                       s, dp, bg, fg, prim, flux, fsig);
+    return;
+  }
   constexpr int H = ReconWidth<RECON>::H;
   constexpr int NP = Layout<MHD>::nprim;
-  const int T = d == 1 ? 2 : 1;
-  const int dt_ = bg.ndim > T;
   const TileShape ts = resolve_tile_shape(d, RECON, MHD, bg, shape);
   if (ts.ts < 0) {
     const unsigned blocks = (unsigned)flux_march_groups(bg, d, ts.ti, -ts.ts);
@@ -392,20 +407,15 @@ static void launch_dir(int d, const DevParams &dp, const BlockGeom &bg, const Pr
     });
     return;
   }
-  const int ts_n = ts.ts, ti_n = ts.ti;
-  const int S = ts_n - 2 * H - 1;
-  const long nic = (bg.ie[0] - bg.is[0] + 3 + ti_n - 1) / ti_n;
-  const long nft = (bg.ie[d] - bg.is[d] + 3 + S - 1) / S;
-  const long ntr = bg.ie[T] - bg.is[T] + 1 + 2 * dt_;
-  const unsigned blocks = (unsigned)(nic * nft * ntr);
-  const int threads = ((ti_n * ts_n + 63) / 64) * 64;
-  const size_t lds = sizeof(double) * (size_t)NP * ts_n * ti_n;
-  if (d == 1)
-    hipLaunchKernelGGL((k_flux_tile<1, RECON, RIEMANN, MHD, GEOM>), dim3(blocks), dim3(threads),
-                       lds, s, dp, bg, ti_n, ts_n, prim, flux, fsig);
-  else
-    hipLaunchKernelGGL((k_flux_tile<2, RECON, RIEMANN, MHD, GEOM>), dim3(blocks), dim3(threads),
-                       lds, s, dp, bg, ti_n, ts_n, prim, flux, fsig);
+  FluxGroups fg{};
+  fg.n[d] = (unsigned)flux_tile_groups(bg, d, ts.ti, ts.ts, H);
+  for (int e = d + 1; e < 4; ++e) fg.off[e] = fg.n[d];
+  fg.ti[d] = ts.ti;
+  fg.ts[d] = ts.ts;
+  const int threads = ((ts.ti * ts.ts + 63) / 64) * 64;
+  const size_t lds = sizeof(double) * (size_t)NP * ts.ts * ts.ti;
+  hipLaunchKernelGGL((k_flux_tile<RECON, RIEMANN, MHD, GEOM>), dim3(fg.n[d]), dim3(threads), lds, s,
+                     dp, bg, fg, prim, flux, fsig);
 }
 
 template <int RECON, int RIEMANN, bool MHD>

@@ -12,6 +12,7 @@
 #include "phx_fixup.h"
 
 #include "phx_device.hpp"
+#include "phx_flux_shapes.hpp"
 
 struct phx_ctx;
 struct phx_mlp;
@@ -73,6 +74,10 @@ void launch_fluxes(int d, int recon, int riemann, int mhd, int geom, const DevPa
                    const BlockGeom &bg, const PrimPtrs &prim, const FluxPtrs &flux, double *fsig,
                    hipStream_t s, TileShape shape, bool fast);
 inline bool flux_fast_of(const phx_fluid_params *p) { return p->flux_arith == PHX_FLUX_ARITH_FAST; }
+// the groups of a launch of every direction at once (launch_fluxes with d = kAllDirs)
+FluxGroups all_flux_groups(int recon, int mhd, const BlockGeom &bg);
+// whether the sweeps of a block whose y/z shapes are not fixed go in one launch
+bool one_launch_fluxes(int recon, int mhd, const BlockGeom &bg);
 // the shape launch_fluxes uses for direction d (after defaults and limits)
 TileShape resolve_tile_shape(int d, int recon, int mhd, const BlockGeom &bg, TileShape want);
 
@@ -300,6 +305,12 @@ struct phx_ctx {
   phx::TileShape tile_for(const phx_fluid_params *p, const phx_block *b, int d) const {
     const auto it = tiles.find(tile_key(p, b, d));
     return it == tiles.end() ? phx::TileShape() : it->second;
+  }
+  // neither y nor z has a shape of its own (autotuned or fixed)
+  bool default_shapes(const phx_fluid_params *p, const phx_block *b) const {
+    for (int d = 1; d < b->ndim; ++d)
+      if (tile_for(p, b, d).ts != 0) return false;
+    return true;
   }
   double *dt_partial = nullptr;  // [kDtPartials]
   std::string last_error;

@@ -772,9 +772,10 @@ int phx_calculate_fluxes(phx_ctx *ctx, const phx_fluid_params *p, const phx_bloc
     return ctx->fail(PHX_ERR_INVALID, "null field");
   const DevParams dp = make_dev_params(p);
   hipStream_t s = ctx->stream_of(stream);
-  for (int d = 0; d < b->ndim; ++d)
+  const bool one = ctx->default_shapes(p, b) && one_launch_fluxes(p->recon, p->mhd, bg);
+  for (int d = one ? kAllDirs : 0; d < (one ? kAllDirs + 1 : b->ndim); ++d)
     launch_fluxes(d, p->recon, p->riemann, p->mhd, p->geom.kind, dp, bg, prim, flux,
-                  f->face_sig, s, ctx->tile_for(p, b, d), flux_fast_of(p));
+                  f->face_sig, s, one ? TileShape() : ctx->tile_for(p, b, d), flux_fast_of(p));
   return ctx->check_launch();
 }
 

@@ -311,11 +311,12 @@ static int fluid_stage_launches(phx_ctx *ctx, const phx_fluid_params *p, const p
   }
   const DevParams dp = make_dev_params(p);
   hipStream_t s = ctx->stream_of(stream);
-  static const char *kFluxName[3] = {"flux_x", "flux_y", "flux_z"};
-  for (int d = 0; d < b->ndim; ++d) {
+  static const char *kFluxName[4] = {"flux_x", "flux_y", "flux_z", "flux_xyz"};
+  const bool one = ctx->default_shapes(p, b) && one_launch_fluxes(p->recon, p->mhd, bg);
+  for (int d = one ? kAllDirs : 0; d < (one ? kAllDirs + 1 : b->ndim); ++d) {
     ctx->mark_begin(kFluxName[d], s);
     launch_fluxes(d, p->recon, p->riemann, p->mhd, p->geom.kind, dp, bg, prim, flux,
-                  f->face_sig, s, ctx->tile_for(p, b, d), flux_fast_of(p));
+                  f->face_sig, s, one ? TileShape() : ctx->tile_for(p, b, d), flux_fast_of(p));
     ctx->mark_end(s);
   }
   if (p->mhd && b->ndim > 1) {  // FluxCT: the EMFs here, the B-flux rewrite in the update

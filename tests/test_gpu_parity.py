@@ -627,6 +627,36 @@ def test_tile_shapes_and_autotune_do_not_change_fluxes(phx, recon, riemann):
     np.testing.assert_array_equal(st.face_sig.get(), first[1])
 
 
+@pytest.mark.parametrize("nx", [(5, 4), (70, 27), (4, 5, 6), (26, 28, 25), (300, 4, 5)])
+@pytest.mark.parametrize("recon,mhd", [(A.RECON_WENO5Z, True), (A.RECON_MP5, False),
+                                       (A.RECON_LINEAR, True), (A.RECON_CONSTANT, False)])
+def test_one_launch_sweeps_match_separate(phx, nx, recon, mhd):
+    """The sweeps of a block in one launch (the default of these sizes: ragged rows, single
+    and several tiles per column, padded group counts) give the bits of the separate
+    launches, and touch nothing outside the face ranges."""
+    say(f"[gpu] one-launch sweeps {nx} recon {recon} mhd {mhd}")
+    rng = np.random.default_rng(len(nx) * 100 + nx[0])
+    b = geom_block(len(nx), nx, A.GEOM_MINKOWSKI)
+    p = fluid_params(gamma=13.0 / 9.0, mhd=mhd, recon=recon, riemann=A.RIEMANN_HLL)
+    prim = random_block(rng, b, mhd, 13.0 / 9.0, A.GEOM_MINKOWSKI)
+    st = BlockState(p, b)
+    st.prim.upload(prim)
+    got = []
+    for shape in ((0, 0), (4, -1)):
+        for d in range(1, len(nx)):
+            phx.set_tile_shape(p, b, d, *shape)
+        st.flux.upload(np.full(st.flux.shape, 7.5))
+        st.face_sig.upload(np.full(st.face_sig.shape, 7.5))
+        phx.calculate_fluxes(p, b, st.fields())
+        synchronize()
+        got.append((st.flux.get(), st.face_sig.get()))
+    for d in range(1, len(nx)):
+        phx.set_tile_shape(p, b, d, 0, 0)
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    assert not np.all(got[0][0] == 7.5)
+
+
 @pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
 def test_sweep_shapes_agree_on_curved_metrics(phx, geom):
     """Tiles and marching waves run the same arithmetic per face, metric included: every
