@@ -198,7 +198,7 @@ void launch_pack_flux(int d, int recon, int riemann, int geom, const DevParams &
                       const PackView &v, long groups, TileShape sh, hipStream_t s);
 }  // namespace flux_fast
 void launch_pack_ct_emf(const PackView &v, long groups, hipStream_t s);
-void launch_pack_sources(int geom, const DevParams &dp, const PackView &v, long groups,
+void launch_pack_sources(int geom, const DevParams &dp, const PackView &v, long groups, int kb,
                          hipStream_t s);
 // The cells a plain con2prim pass leaves to the learned bracket: those with no previous
 // root (mu <= 0: initial data, fresh cells).  Entries are (block << 32) | (keep << 31) |
@@ -268,6 +268,8 @@ void launch_pack_floors(int geom, const DevParams &dp, const DevFixup &fx, const
 void launch_geo_fill(const DevParams &dp, const BlockGeom &bg, double *geo, hipStream_t s);
 // groups per block for each launch kind
 long pack_groups_flux(int d, int recon, const BlockGeom &bg, TileShape shape);
+int source_cells(long cells);  // cells along x3 per lane of the source kernels
+long pack_groups_sources(const BlockGeom &bg, int kb);
 long pack_groups_cells(const BlockGeom &bg, bool corners);
 
 // partial minima of the CFL reduction (one per 256-cell block of the fused stage kernel,

@@ -396,23 +396,11 @@ void launch_geo_fill(const DevParams &dp, const BlockGeom &bg, double *geo, hipS
   hipLaunchKernelGGL(k_geo_fill, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, dp, bg, geo);
 }
 
-// geometric source terms of interior cell t of block b
-template <bool MHD, int GEOM, bool CACHED = false, class PP, class SP>
-__device__ __forceinline__ void sources_body(const DevParams &p, const BlockGeom &b, long t,
-                                             const PP &prim, const SP &src) {
+// geometric source terms of cell c at metric g with derivatives dv
+template <bool MHD, class M, class PP, class SP>
+__device__ __forceinline__ void sources_cell(const M &g, const KSDerivs &dv, long c, const PP &prim,
+                                             const SP &src) {
   using L = Layout<MHD>;
-  using M = typename MetricOf<GEOM>::type;
-  const int ni = b.ie[0] - b.is[0] + 1, nj = b.ie[1] - b.is[1] + 1, nk = b.ie[2] - b.is[2] + 1;
-  if (t >= (long)ni * nj * nk) return;
-  const int i = (int)(t % ni) + b.is[0];
-  const int j = (int)((t / ni) % nj) + b.is[1];
-  const int k = (int)(t / ((long)ni * nj)) + b.is[2];
-  const long c = ((long)k * b.nj + j) * b.ni + i;
-  const double X1 = xc(b, 0, i), X2 = xc(b, 1, j), X3 = xc(b, 2, k);
-  const long q = (long)j * b.ni + i;
-  const M g = metric_at<GEOM, CACHED>(p, b, 0, q, X1, X2, X3);
-  KSDerivs dv;
-  geom_derivs_at<GEOM, CACHED>(p, b, q, X1, X2, X3, dv);
   double pr[L::nprim];
   for (int v = 0; v < L::nprim; ++v) pr[v] = prim[v][c];
   // tmunu.hpp:94-126
@@ -481,10 +469,34 @@ __device__ __forceinline__ void sources_body(const DevParams &p, const BlockGeom
   src[4][c] = gdet * alpha * (Ta - TGam);
 }
 
+// geometric source terms of kb interior cells of block b along x3: column t % (nx ny), cells
+// (t / (nx ny)) kb and on.  Neither metric depends on X3, so the metric, its derivatives and
+// g^{mu nu} (51 numbers from the cached plane, or five metric evaluations) are had once for the
+// kb cells (source_cells)
+template <bool MHD, int GEOM, bool CACHED = false, class PP, class SP>
+__device__ __forceinline__ void sources_body(const DevParams &p, const BlockGeom &b, long t, int kb,
+                                             const PP &prim, const SP &src) {
+  using M = typename MetricOf<GEOM>::type;
+  const int ni = b.ie[0] - b.is[0] + 1, nj = b.ie[1] - b.is[1] + 1, nk = b.ie[2] - b.is[2] + 1;
+  if (t >= (long)ni * nj * ((nk + kb - 1) / kb)) return;
+  const int i = (int)(t % ni) + b.is[0];
+  const int j = (int)((t / ni) % nj) + b.is[1];
+  const int k0 = (int)(t / ((long)ni * nj)) * kb + b.is[2];
+  const double X1 = xc(b, 0, i), X2 = xc(b, 1, j), X3 = xc(b, 2, k0);
+  const long q = (long)j * b.ni + i;
+  const M g = metric_at<GEOM, CACHED>(p, b, 0, q, X1, X2, X3);
+  KSDerivs dv;
+  geom_derivs_at<GEOM, CACHED>(p, b, q, X1, X2, X3, dv);
+  const int k1 = min(k0 + kb - 1, b.ie[2]);
+#pragma unroll 1
+  for (int k = k0; k <= k1; ++k)
+    sources_cell<MHD>(g, dv, ((long)k * b.nj + j) * b.ni + i, prim, src);
+}
+
 template <bool MHD, int GEOM>
-__global__ __launch_bounds__(128) void k_sources(DevParams p, BlockGeom b, PrimPtrs prim,
+__global__ __launch_bounds__(128) void k_sources(DevParams p, BlockGeom b, int kb, PrimPtrs prim,
                                                  ConsPtrs src) {
-  sources_body<MHD, GEOM>(p, b, (long)blockIdx.x * blockDim.x + threadIdx.x, prim, src);
+  sources_body<MHD, GEOM>(p, b, (long)blockIdx.x * blockDim.x + threadIdx.x, kb, prim, src);
 }
 
 template <int NC>
@@ -505,17 +517,13 @@ __global__ __launch_bounds__(256) void k_pack_ct_emf(PackView v) {
 }
 
 template <int GEOM>
-__global__ __launch_bounds__(128) void k_pack_sources(DevParams p, PackView v) {
+__global__ __launch_bounds__(128) void k_pack_sources(DevParams p, PackView v, int kb) {
   const long g = xcd_remap(blockIdx.x, gridDim.x);
   const int b = pack_find(v.start, v.n, g);
   const PackEntry &E = v.e[b];
-  // two 128-thread halves per 256-cell group
   const Contig prim = contig(E.prim, E.bg.ncell), src = contig(E.src, E.bg.ncell);
-  sources_body<true, GEOM, GEOM == PHX_GEOM_FMKS>(p, E.bg, (g - v.start[b]) * 256 + threadIdx.x,
-                                                 prim, src);
-  sources_body<true, GEOM, GEOM == PHX_GEOM_FMKS>(p, E.bg,
-                                                 (g - v.start[b]) * 256 + 128 + threadIdx.x,
-                                                 prim, src);
+  sources_body<true, GEOM, GEOM == PHX_GEOM_FMKS>(p, E.bg, (g - v.start[b]) * 128 + threadIdx.x,
+                                                 kb, prim, src);
 }
 
 // ---- batched con2prim / prim2con over independent states --------------------------------
@@ -666,6 +674,28 @@ int check_block(phx_ctx *ctx, const phx_block *b, int recon) {
   return PHX_OK;
 }
 
+// Cells along x3 per lane of the source kernels over a block or pack of this many cells: the
+// fewest that leave no more waves than are resident at once, two per SIMD with the metrics'
+// registers.  A lane's time is that of its metric and derivatives (five metric evaluations on
+// FMKS without a plane, 51 loads with it), which a few cells hardly lengthen, so a second round
+// of waves costs more than cells in a lane do; within one round each further cell adds 0.7 us to
+// the latency.  us at 1 / 2 / 4 / 8 cells, FMKS: 32^3 21.7 / 22.7 / 24.7 / 29.0, 64x64x32
+// 28.2 / 28.5 / 26.2 / 29.9, 64^3 49.2 / 31.1 / 32.5 / 31.7, 72^3 72.5 / 48.4 / 37.6 / 42.7;
+// Kerr-Schild: 64^3 17.1 / 15.0 / 17.2 / 18.4, 72^3 22.9 / 20.0 / 18.8 / 24.2; a pack of 2.1 M
+// cells from the FMKS plane 103 / - / 71.5 / 71.8.
+int source_cells(long cells) {
+  int kb = 1;
+  while (kb < 4 && cells > 2048L * 64 * kb) kb *= 2;
+  return kb;
+}
+
+// 128-lane groups of the pack's source kernel
+long pack_groups_sources(const BlockGeom &bg, int kb) {
+  const long n = (long)(bg.ie[0] - bg.is[0] + 1) * (bg.ie[1] - bg.is[1] + 1) *
+                 ((bg.ie[2] - bg.is[2] + kb) / kb);
+  return (n + 127) / 128;
+}
+
 long pack_groups_cells(const BlockGeom &bg, bool corners) {
   const long c = corners ? 1 : 0;
   const long n = (bg.ie[0] - bg.is[0] + 1 + c) * (bg.ie[1] - bg.is[1] + 1 + c) *
@@ -673,13 +703,14 @@ long pack_groups_cells(const BlockGeom &bg, bool corners) {
   return (n + 255) / 256;
 }
 
-void launch_pack_sources(int geom, const DevParams &dp, const PackView &v, long groups,
+void launch_pack_sources(int geom, const DevParams &dp, const PackView &v, long groups, int kb,
                          hipStream_t s) {
   if (groups <= 0) return;
   with_geom(geom, [&](auto G) {
     constexpr int GEOM = decltype(G)::value;
     if constexpr (GEOM != PHX_GEOM_MINKOWSKI)
-      hipLaunchKernelGGL((k_pack_sources<GEOM>), dim3((unsigned)groups), dim3(128), 0, s, dp, v);
+      hipLaunchKernelGGL((k_pack_sources<GEOM>), dim3((unsigned)groups), dim3(128), 0, s, dp, v,
+                         kb);
   });
 }
 
@@ -723,13 +754,16 @@ void launch_sources(int geom, int mhd, const DevParams &dp, const BlockGeom &bg,
       hipLaunchKernelGGL(k_zero_sources<5>, dim3(nblocks(bg.ncell, 256)), dim3(256), 0, s, bg, src);
     return;
   }
-  const long n = (long)(bg.ie[0] - bg.is[0] + 1) * (bg.ie[1] - bg.is[1] + 1) * (bg.ie[2] - bg.is[2] + 1);
+  const long cols = (long)(bg.ie[0] - bg.is[0] + 1) * (bg.ie[1] - bg.is[1] + 1);
+  const int nk = bg.ie[2] - bg.is[2] + 1;
+  const int kb = source_cells(cols * nk);
+  const long n = cols * ((nk + kb - 1) / kb);
   with_geom(geom, [&](auto G) {
     constexpr int GEOM = decltype(G)::value;
     if constexpr (GEOM != PHX_GEOM_MINKOWSKI)
       with_mhd(mhd, [&](auto H) {
         hipLaunchKernelGGL((k_sources<decltype(H)::value, GEOM>), dim3(nblocks(n, 128)), dim3(128),
-                           0, s, dp, bg, prim, src);
+                           0, s, dp, bg, kb, prim, src);
       });
   });
 }

@@ -59,7 +59,8 @@ int build_start(phx_pack *k, int kind) {
                    : kind < 5 ? pack_groups_cells(g, kind == 3)
                    : kind == 5 ? (g.ncell + 255) / 256
                    : kind == 6 ? (nf + 255) / 256
-                               : (g.ncell - nint + 255) / 256;
+                   : kind == 7 ? (g.ncell - nint + 255) / 256
+                               : pack_groups_sources(g, k->src_cells);
     st[b + 1] = st[b] + c;
   }
   if (st[k->n] > (long)UINT_MAX) return PHX_ERR_INVALID;
@@ -94,7 +95,8 @@ void launch_stage_fluxes(phx_ctx *ctx, phx_pack *k, int st, hipStream_t s) {
   ctx->mark_end(s);
   if (k->p.geom.kind != PHX_GEOM_MINKOWSKI) {
     ctx->mark_begin("sources", s);
-    launch_pack_sources(k->p.geom.kind, k->dp, view(k, st, 4), k->groups[4], s);
+    launch_pack_sources(k->p.geom.kind, k->dp, view(k, st, 8), k->groups[8], k->src_cells,
+                        s);
     ctx->mark_end(s);
   }
 }
@@ -227,7 +229,11 @@ int phx_pack_create(phx_ctx *ctx, const phx_fluid_params *p, int nblocks,
     ok = hipMalloc(&k->entries[st], sizeof(PackEntry) * nblocks) == hipSuccess &&
          hipMemcpy(k->entries[st], e[st].data(), sizeof(PackEntry) * nblocks,
                    hipMemcpyHostToDevice) == hipSuccess;
-  for (int kind = 0; kind < 8 && ok; ++kind) ok = build_start(k, kind) == PHX_OK;
+  long cells = 0;
+  for (const BlockGeom &g : k->geoms)
+    cells += (long)(g.ie[0] - g.is[0] + 1) * (g.ie[1] - g.is[1] + 1) * (g.ie[2] - g.is[2] + 1);
+  k->src_cells = source_cells(cells);
+  for (int kind = 0; kind < 9 && ok; ++kind) ok = build_start(k, kind) == PHX_OK;
   ok = ok && hipMalloc(&k->partial, sizeof(double) * std::max({k->groups[4] + 1, k->groups[5], 1L})) ==
                  hipSuccess;
   ok = ok && hipMalloc(&k->counters, 2 * sizeof(unsigned long long)) == hipSuccess &&

@@ -658,6 +658,37 @@ def test_one_launch_sweeps_match_separate(phx, nx, recon, mhd):
 
 
 @pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
+@pytest.mark.parametrize("nx,mhd", [((64, 64, 33), True), ((72, 72, 51), True),
+                                    ((72, 72, 50), False)])
+def test_sources_of_several_cells_per_lane(phx, geom, nx, mhd):
+    """Blocks whose lanes take two and four cells along x3, with a remainder at the end, give
+    the bits of blocks of three layers, whose lanes take one, in every layer."""
+    say(f"[gpu] sources geom {geom} {nx} mhd {mhd}")
+    rng = np.random.default_rng(nx[2])
+    b = geom_block(3, nx, geom)
+    p = geom_params(geom, gamma=13.0 / 9.0, mhd=mhd, recon=A.RECON_WENO5Z,
+                    riemann=A.RIEMANN_HLL)
+    prim = random_block(rng, b, mhd, 13.0 / 9.0, geom)
+    st = BlockState(p, b)
+    st.prim.upload(prim)
+    st.src.upload(np.full(st.src.shape, 7.5))
+    phx.fluid_source_terms(p, b, st.fields(with_src=True))
+    synchronize()
+    got, ng = st.src.get(), b.ng
+    inner = (slice(None), slice(None), slice(ng, ng + nx[1]), slice(ng, ng + nx[0]))
+    thin = geom_block(3, nx[:2] + (3,), geom)
+    ts = BlockState(p, thin)
+    for k in range(0, nx[2] - 2, 3):
+        k = k if k + 6 <= nx[2] else nx[2] - 3
+        ts.prim.upload(np.ascontiguousarray(prim[:, k:k + 3 + 2 * ng]))
+        phx.fluid_source_terms(p, thin, ts.fields(with_src=True))
+        synchronize()
+        np.testing.assert_array_equal(got[inner][1:5, ng + k:ng + k + 3],
+                                      ts.src.get()[inner][1:5, ng:ng + 3])
+    assert np.all(got[1:5, :ng] == 7.5) and np.all(got[1:5, ng + nx[2]:] == 7.5)
+
+
+@pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
 def test_sweep_shapes_agree_on_curved_metrics(phx, geom):
     """Tiles and marching waves run the same arithmetic per face, metric included: every
     shape gives the same bits on Kerr-Schild and FMKS blocks (the oracle bars for these
