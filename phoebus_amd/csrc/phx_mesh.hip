@@ -34,91 +34,26 @@ __device__ __forceinline__ void block_loc(const MeshInfo &m, int gid, int lx[3])
   lx[2] = gid / (m.nb[0] * m.nb[1]);
 }
 
-// the FillGhost fields of a cell (bc_vars = primitive, fluid.cpp:159-165): primitives,
-// temperature, con2prim root, fail flag and the conserved variables of the container
+// Every ghost cell of the mesh in one pass.  The FillGhost fields (bc_vars = primitive,
+// fluid.cpp:159-165: primitives, temperature, con2prim root, fail flag and the conserved
+// variables of the container) come from one interior cell: the owner of the ghost's mesh index
+// after the periodic wrap (parthenon's same-level ghost fill), with the index clamped to the
+// mesh in a gr_outflow dimension (OutflowInnerX1 / OuterX1, phoebus_boundaries.cpp:118-152,
+// 222-262; GenericBC outflow for x2, x3, :43-116).  Filling the faces in the order x1, x2, x3
+// over the entire extent of the other dimensions ends in the same cell.  Sources are interior
+// cells and destinations ghosts, so no order among the lanes matters.
+// ConvertBoundaryConditions (phoebus_boundaries.cpp:303-448) is part of it: on the ghost slabs
+// of every face that is not a block boundary (physical or periodic mesh faces), the FMKS
+// outer-x1 inflow check (:356-380: no u^1 < 0 inflow from the outer boundary), then p2c into the
+// container and the cell signal speeds, from the primitives in hand; such a cell's conserved
+// variables are not copied.
+// Bound by the gathers: a ghost's 13 to 21 fields read and 16 to 24 written, x1 ghosts in runs
+// of ng cells.  35 us for the 395,000 ghosts of a 128x64x64 torus mesh; a pass for the exchange,
+// one for each outflow dimension (which copied the exchange's ghosts again) and one for the
+// conversion, which read the primitives again, took 36 us more.
 constexpr int kNprim = 10, kNcons = 8;
-// (all 21 values are read before any is written: the source and destination fields share
-// one allocation as far as the compiler can tell, so interleaved copies would each wait a
-// full memory round trip)
-__device__ __forceinline__ void copy_ghost_fields(const PackEntry &D, long cd, const PackEntry &S,
-                                                  long cs) {
-  const long nd = D.bg.ncell, ns = S.bg.ncell;
-  double pr[kNprim], u[kNcons];
-#pragma unroll
-  for (int v = 0; v < kNprim; ++v) pr[v] = S.prim_out[v * ns + cs];
-#pragma unroll
-  for (int v = 0; v < kNcons; ++v) u[v] = S.u_out[v * ns + cs];
-  const double t = D.temp ? S.temp[cs] : 0.0, m = S.mu[cs], f = S.fail[cs];
-#pragma unroll
-  for (int v = 0; v < kNprim; ++v) D.prim_out[v * nd + cd] = pr[v];
-#pragma unroll
-  for (int v = 0; v < kNcons; ++v) D.u_out[v * nd + cd] = u[v];
-  if (D.temp) D.temp[cd] = t;
-  D.mu[cd] = m;
-  D.fail[cd] = f;
-}
-
-// boundary exchange between blocks of one level (parthenon's same-level ghost fill): a
-// ghost cell whose mesh index lies inside the mesh, after the periodic wrap, takes the
-// fields of the block that owns that index; the others are left to the physical boundaries
-__global__ __launch_bounds__(256) void k_mesh_exchange(MeshInfo m, PackView v) {
-  const long g = xcd_remap(blockIdx.x, gridDim.x);
-  const int b = pack_find(v.start, v.n, g);
-  const PackEntry &E = v.e[b];
-  int idx[3];
-  if (!ghost_cell(E.bg, (g - v.start[b]) * 256 + threadIdx.x, idx)) return;
-  int lx[3];
-  block_loc(m, b, lx);
-  int src[3], sl[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    int gi = lx[d] * m.bnx[d] + idx[d] - m.ng;
-    if (gi < 0 || gi >= m.N[d]) {
-      if (!m.periodic[d]) return;
-      gi = gi < 0 ? gi + m.N[d] : gi - m.N[d];
-    }
-    src[d] = gi / m.bnx[d];
-    sl[d] = gi % m.bnx[d] + m.ng;
-  }
-  const PackEntry &S = v.e[src[0] + m.nb[0] * (src[1] + m.nb[1] * src[2])];
-  const long cd = ((long)idx[2] * E.bg.nj + idx[1]) * E.bg.ni + idx[0];
-  const long cs = ((long)sl[2] * S.bg.nj + sl[1]) * S.bg.ni + sl[0];
-  copy_ghost_fields(E, cd, S, cs);
-}
-
-// gr_outflow with bc_vars = primitive (OutflowInnerX1 / OuterX1, phoebus_boundaries.cpp:
-// 118-152, 222-262; GenericBC outflow for x2, x3, :43-116): the ghost slab of a physical
-// face of dimension d copies the first (last) interior layer, all FillGhost fields, over
-// the entire extent of the other dimensions
-__global__ __launch_bounds__(256) void k_mesh_outflow(MeshInfo m, PackView v, int d, int inner,
-                                                      int outer) {
-  const long g = xcd_remap(blockIdx.x, gridDim.x);
-  const int b = pack_find(v.start, v.n, g);
-  int lx[3];
-  block_loc(m, b, lx);
-  // a block on neither physical face of d has nothing to do (the whole workgroup)
-  if (!(inner && lx[d] == 0) && !(outer && lx[d] == m.nb[d] - 1)) return;
-  const PackEntry &E = v.e[b];
-  int idx[3];
-  if (!ghost_cell(E.bg, (g - v.start[b]) * 256 + threadIdx.x, idx)) return;
-  int ref[3] = {idx[0], idx[1], idx[2]};
-  if (idx[d] < E.bg.is[d] && inner && lx[d] == 0)
-    ref[d] = E.bg.is[d];
-  else if (idx[d] > E.bg.ie[d] && outer && lx[d] == m.nb[d] - 1)
-    ref[d] = E.bg.ie[d];
-  else
-    return;
-  const long c = ((long)idx[2] * E.bg.nj + idx[1]) * E.bg.ni + idx[0];
-  const long cr = ((long)ref[2] * E.bg.nj + ref[1]) * E.bg.ni + ref[0];
-  copy_ghost_fields(E, c, E, cr);
-}
-
-// ConvertBoundaryConditions (phoebus_boundaries.cpp:303-448) for bc_vars = primitive: on
-// the ghost slabs of every face that is not a block boundary (physical or periodic mesh
-// faces), the FMKS outer-x1 inflow check (:356-380: no u^1 < 0 inflow from the outer
-// boundary), then p2c into the container and the cell signal speeds
 template <int GEOM>
-__global__ __launch_bounds__(256) void k_mesh_convert(DevParams p, MeshInfo m, PackView v) {
+__global__ __launch_bounds__(256) void k_mesh_fill_ghosts(DevParams p, MeshInfo m, PackView v) {
   using M = typename MetricOf<GEOM>::type;
   const long g = xcd_remap(blockIdx.x, gridDim.x);
   const int b = pack_find(v.start, v.n, g);
@@ -128,44 +63,74 @@ __global__ __launch_bounds__(256) void k_mesh_convert(DevParams p, MeshInfo m, P
   if (!ghost_cell(bg, (g - v.start[b]) * 256 + threadIdx.x, idx)) return;
   int lx[3];
   block_loc(m, b, lx);
+  int src[3], sl[3];
   bool slab = false, outer_x1 = false;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    if (idx[d] < bg.is[d] && lx[d] == 0) slab = true;
-    if (idx[d] > bg.ie[d] && lx[d] == m.nb[d] - 1) {
+    int gi = lx[d] * m.bnx[d] + idx[d] - m.ng;
+    if (gi < 0 || gi >= m.N[d]) {
       slab = true;
-      if (d == 0) outer_x1 = true;
+      if (d == 0) outer_x1 = gi >= m.N[d];
+      if (m.periodic[d])
+        gi = gi < 0 ? gi + m.N[d] : gi - m.N[d];
+      else
+        gi = gi < 0 ? 0 : m.N[d] - 1;
     }
+    src[d] = gi / m.bnx[d];
+    sl[d] = gi % m.bnx[d] + m.ng;
   }
-  if (!slab) return;
-  const long n = bg.ncell, c = ((long)idx[2] * bg.nj + idx[1]) * bg.ni + idx[0];
-  if constexpr (GEOM == PHX_GEOM_FMKS) {
-    if (outer_x1 && m.inflow) {
-      const M gm = metric_at<GEOM, true>(p, bg, 0, (long)idx[1] * bg.ni + idx[0],
-                                         xc(bg, 0, idx[0]), xc(bg, 1, idx[1]), xc(bg, 2, idx[2]));
-      double vcon[3] = {E.prim_out[n + c], E.prim_out[2 * n + c], E.prim_out[3 * n + c]};
-      double W = lorentz_factor(gm, vcon);
-      const double alpha = gm.alpha(), beta0 = gm.beta(0);
-      const double ucon1 = vcon[0] - W * beta0 / alpha;
-      if (ucon1 < 0) {
+  const PackEntry &S = v.e[src[0] + m.nb[0] * (src[1] + m.nb[1] * src[2])];
+  const long c = ((long)idx[2] * bg.nj + idx[1]) * bg.ni + idx[0], n = bg.ncell;
+  const long cs = ((long)sl[2] * S.bg.nj + sl[1]) * S.bg.ni + sl[0], ns = S.bg.ncell;
+  // (all values are read before any is written: the source and destination fields share one
+  // allocation as far as the compiler can tell, so interleaved copies would each wait a full
+  // memory round trip)
+  double pr[kNprim], u[kNcons];
 #pragma unroll
-        for (int ii = 0; ii < 3; ++ii) vcon[ii] /= W;
-        vcon[0] = beta0 / alpha;
-        double vsq = 0.;
+  for (int q = 0; q < kNprim; ++q) pr[q] = S.prim_out[q * ns + cs];
+  const double t = S.temp ? S.temp[cs] : 0.0, mu = S.mu[cs], f = S.fail[cs];
+  if (slab) {
+    const M gm = metric_at<GEOM, GEOM == PHX_GEOM_FMKS>(p, bg, 0, (long)idx[1] * bg.ni + idx[0],
+                                                        xc(bg, 0, idx[0]), xc(bg, 1, idx[1]),
+                                                        xc(bg, 2, idx[2]));
+    if constexpr (GEOM == PHX_GEOM_FMKS) {
+      if (outer_x1 && m.inflow) {
+        double vcon[3] = {pr[1], pr[2], pr[3]};
+        double W = lorentz_factor(gm, vcon);
+        const double alpha = gm.alpha(), beta0 = gm.beta(0);
+        const double ucon1 = vcon[0] - W * beta0 / alpha;
+        if (ucon1 < 0) {
 #pragma unroll
-        for (int ii = 0; ii < 3; ++ii)
+          for (int ii = 0; ii < 3; ++ii) vcon[ii] /= W;
+          vcon[0] = beta0 / alpha;
+          double vsq = 0.;
 #pragma unroll
-          for (int jj = 0; jj < 3; ++jj)
-            if (M::nz_cov(ii + 1, jj + 1)) vsq += gm.gcov(ii + 1, jj + 1) * vcon[ii] * vcon[jj];
-        W = 1. / sqrt(1. - vsq);
+          for (int ii = 0; ii < 3; ++ii)
 #pragma unroll
-        for (int ii = 0; ii < 3; ++ii) E.prim_out[(1 + ii) * n + c] = W * vcon[ii];
+            for (int jj = 0; jj < 3; ++jj)
+              if (M::nz_cov(ii + 1, jj + 1)) vsq += gm.gcov(ii + 1, jj + 1) * vcon[ii] * vcon[jj];
+          W = 1. / sqrt(1. - vsq);
+#pragma unroll
+          for (int ii = 0; ii < 3; ++ii) pr[1 + ii] = W * vcon[ii];
+        }
       }
     }
+    const double vp[3] = {pr[1], pr[2], pr[3]}, bp[3] = {pr[5], pr[6], pr[7]};
+    double sig[3];
+    p2c<true>(pr[0], vp, bp, pr[4], pr[8], pr[9], gm, u[0], u + 1, u + 5, u[4], sig);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) E.csig[d * n + c] = sig[d];
+  } else {
+#pragma unroll
+    for (int q = 0; q < kNcons; ++q) u[q] = S.u_out[q * ns + cs];
   }
-  prim_to_con_cell<true, GEOM, GEOM == PHX_GEOM_FMKS>(
-      p, bg, idx[0], idx[1], idx[2], contig(E.prim_out, bg.ncell), contig(E.u_out, bg.ncell),
-      E.csig);
+#pragma unroll
+  for (int q = 0; q < kNprim; ++q) E.prim_out[q * n + c] = pr[q];
+#pragma unroll
+  for (int q = 0; q < kNcons; ++q) E.u_out[q * n + c] = u[q];
+  if (E.temp) E.temp[c] = t;
+  E.mu[c] = mu;
+  E.fail[c] = f;
 }
 
 // FixFluxes for gr_outflow (fixup.cpp:759-1062): no mass inflow through a physical face,
@@ -278,29 +243,15 @@ long groups(const phx_mesh *m, int kind) { return m->pack->groups[kind]; }
 
 void launch_exchange_and_boundaries(phx_mesh *m, int st, hipStream_t s) {
   phx_ctx *ctx = m->ctx;
-  // every kernel here writes ghost cells only: a work list of them
-  const PackView v = pv(m, st, 7);
-  const unsigned gr = (unsigned)groups(m, 7);
-  ctx->mark_begin("exchange", s);
-  hipLaunchKernelGGL(k_mesh_exchange, dim3(gr), dim3(256), 0, s, m->mi, v);
-  ctx->mark_end(s);
-  // ApplyBoundaryConditions: faces in the order inner/outer x1, x2, x3
-  for (int d = 0; d < 3; ++d) {
-    const int inner = m->outflow_mask >> (2 * d) & 1, outer = m->outflow_mask >> (2 * d + 1) & 1;
-    if (!inner && !outer) continue;
-    ctx->mark_begin("outflow", s);
-    hipLaunchKernelGGL(k_mesh_outflow, dim3(gr), dim3(256), 0, s, m->mi, v, d, inner, outer);
-    ctx->mark_end(s);
-  }
-  ctx->mark_begin("convert", s);
+  const PackView v = pv(m, st, 7);  // ghost cells only
+  ctx->mark_begin("fill_ghosts", s);
   with_geom(m->p.geom.kind, [&](auto G) {
-    hipLaunchKernelGGL((k_mesh_convert<decltype(G)::value>), dim3(gr), dim3(256), 0, s,
-                       m->pack->dp, m->mi, v);
+    hipLaunchKernelGGL((k_mesh_fill_ghosts<decltype(G)::value>), dim3((unsigned)groups(m, 7)),
+                       dim3(256), 0, s, m->pack->dp, m->mi, v);
   });
   ctx->mark_end(s);
 }
 
-// the learned-bracket pass over the cells queued since the queue was last cleared
 void launch_c2p_queued(phx_mesh *m, int st, const char *name, hipStream_t s) {
   phx_pack *k = m->pack;
   m->ctx->mark_begin(name, s);

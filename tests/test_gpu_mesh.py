@@ -99,6 +99,39 @@ def test_minkowski_mesh_bit_exact(phx, case):
     m.close()
 
 
+O_, P_ = A.BC_OUTFLOW, A.BC_PERIODIC
+
+
+@pytest.mark.parametrize("N,bnx,bc", [
+    ((8, 4, 16), (4, 4, 8), (O_, O_, P_, P_, O_, O_)),   # one block wide, wrapping onto itself
+    ((10, 16, 8), (5, 4, 8), (O_,) * 6),                 # corners clamped in all dimensions
+    ((4, 8, 12), (4, 8, 4), (P_, P_, O_, O_, P_, P_)),
+])
+def test_ghost_fill_of_narrow_blocks_bit_exact(phx, N, bnx, bc):
+    """Blocks as narrow as their ghost zones, every mix of wrapped, clamped and neighbouring
+    sources in edges and corners: the entire blocks hold the oracle mesh's bits."""
+    say(f"[gpu] mesh {N} in blocks of {bnx}, boundaries {bc}, vs oracle mesh")
+    xmax = tuple(n / 16 for n in N)
+    p = fluid_params(gamma=4 / 3, mhd=True, recon=A.RECON_WENO5Z, riemann=A.RIEMANN_HLL,
+                     c2p_tol=1e-10)
+    op = O.default_params(gamma=4 / 3, mhd=True, recon=O.RECON_WENO5, riemann=O.RIEMANN_HLL,
+                          tol=1e-10)
+    m = Mesh(phx, p, N, bnx, (0, 0, 0), xmax, bc, cfl=0.3)
+    om = O.MeshDriver(op, N, bnx, (0, 0, 0), xmax, bc, cfl=0.3)
+    G = _wave_prims(N, 4, (0, 0, 0), xmax)
+    for g, pr in _blocks_of(G, om.loc, bnx):
+        m.set_prim(g, pr)
+        om.set_prim(g, pr)
+    m.initialize()
+    om.initialize()
+    _compare(m, om, True, "initial")
+    for s in range(2):
+        m.step()
+        om.step()
+        _compare(m, om, True, f"step {s + 1}")
+    m.close()
+
+
 def test_fmks_torus_mesh_to_solver_tolerance(phx):
     say("[gpu] FMKS torus mesh 32x16x8 in 4 blocks vs oracle mesh")
     N, bnx = (32, 16, 8), (16, 8, 8)
