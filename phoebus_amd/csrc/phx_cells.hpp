@@ -119,22 +119,21 @@ __device__ __forceinline__ double eos_bmod_rho_sie(const DevParams &p, double rh
   return (p.gm1 + 1.0) * p.gm1 * rho * sie;
 }
 
-// con2prim of cell c = (i, j, k) of block b, in place on cons / prim / temp / mu / csig;
-// writes the fail flag and the iteration count
+// con2prim of cell c = (i, j, k) of block b, in place on cons / prim / temp / mu / csig, from
+// the conserved variables in cs, which cons holds too; writes the fail flag and the iteration
+// count
 template <bool MHD, int GEOM, bool CACHED = false, class CP, class PP>
-__device__ __forceinline__ void con2prim_cell(const DevParams &p, const BlockGeom &b, int i,
-                                              int j, int k, const CP &cons, const PP &prim,
-                                              double *__restrict__ temp,
-                                              double *__restrict__ mu,
-                                              double *__restrict__ csig,
-                                              double *__restrict__ fail,
-                                              int32_t *__restrict__ iters) {
-  using L = Layout<MHD>;
+__device__ __forceinline__ void con2prim_loaded(const DevParams &p, const BlockGeom &b, int i,
+                                                int j, int k, double cs[Layout<MHD>::ncons],
+                                                const CP &cons, const PP &prim,
+                                                double *__restrict__ temp,
+                                                double *__restrict__ mu,
+                                                double *__restrict__ csig,
+                                                double *__restrict__ fail,
+                                                int32_t *__restrict__ iters) {
   const long c = ((long)k * b.nj + j) * b.ni + i;
   const long n = b.ncell;
-  double cs[L::ncons], sig[3];
-#pragma unroll
-  for (int v = 0; v < L::ncons; ++v) cs[v] = cons[v][c];
+  double sig[3];
   // zones rejected up front by the NaN test keep every field (con2prim_robust.hpp:303-304)
   if (isnan(cs[0]) + isnan(cs[1]) + isnan(cs[4]) > 0) {
     fail[c] = 0.0;
@@ -151,6 +150,22 @@ __device__ __forceinline__ void con2prim_cell(const DevParams &p, const BlockGeo
     if (solved && d < b.ndim) csig[d * n + c] = sig[d];
   fail[c] = st;
   if (iters) iters[c] = it;
+}
+
+template <bool MHD, int GEOM, bool CACHED = false, class CP, class PP>
+__device__ __forceinline__ void con2prim_cell(const DevParams &p, const BlockGeom &b, int i,
+                                              int j, int k, const CP &cons, const PP &prim,
+                                              double *__restrict__ temp,
+                                              double *__restrict__ mu,
+                                              double *__restrict__ csig,
+                                              double *__restrict__ fail,
+                                              int32_t *__restrict__ iters) {
+  using L = Layout<MHD>;
+  const long c = ((long)k * b.nj + j) * b.ni + i;
+  double cs[L::ncons];
+#pragma unroll
+  for (int v = 0; v < L::ncons; ++v) cs[v] = cons[v][c];
+  con2prim_loaded<MHD, GEOM, CACHED>(p, b, i, j, k, cs, cons, prim, temp, mu, csig, fail, iters);
 }
 
 // p2c of cell (i, j, k): cons (with B) and, when csig is given, the cell signal speeds

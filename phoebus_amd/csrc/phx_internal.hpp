@@ -144,6 +144,13 @@ int check_block(phx_ctx *ctx, const phx_block *b, int recon);
 void launch_flux_ct(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s);
 // FluxCT's corner EMFs alone (the fused updates form the rewritten B fluxes from them)
 void launch_ct_emf(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s);
+// the update of the interior (beta, dt as in phx_flux_divergence_update; with MHD in 2-D and 3-D
+// the magnetic fluxes from the corner EMFs) and the con2prim of the entire block on u_out
+void launch_update_con2prim_entire(const phx_fluid_params &p, const BlockGeom &bg, int ndim,
+                                   const FluxPtrs &flux, const double *emf, const ConsPtrs &src,
+                                   const ConsPtrs &u_stage, const ConsPtrs &u_base, double beta,
+                                   double dt, const ConsPtrs &u_out, const PrimPtrs &prim_out,
+                                   const phx_block_fields &f, int32_t *iters, hipStream_t s);
 void launch_sources(int geom, int mhd, const DevParams &dp, const BlockGeom &bg,
                     const PrimPtrs &prim, const ConsPtrs &src, hipStream_t s);
 void launch_dt_finish(const double *partial, int np, double cfl, double *dt, hipStream_t s);

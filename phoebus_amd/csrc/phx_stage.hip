@@ -11,6 +11,7 @@
 #include <mutex>
 
 #include "phx.h"
+#include "phx_cells.hpp"
 #include "phx_device.hpp"
 #include "phx_internal.hpp"
 
@@ -73,9 +74,62 @@ __device__ __forceinline__ void face_fluxes(const FP &flux, const double *__rest
   }
 }
 
+// dU/dt of cell c from its face fluxes, the average into U_s and U_{s+1} into u_out and cs.
+// CT: take the magnetic fluxes from the corner EMFs in emf (face_fluxes) instead of flux.
+// parthenon FluxDivergence (uniform coordinates), SumData, AverageIndependentData,
+// UpdateIndependentData -- the operation order of the separate kernels
+template <bool MHD, int GEOM, int NDIM, bool CT, class FP, class CP>
+__device__ __forceinline__ void update_cell(const BlockGeom &b, long c, const FP &flux,
+                                            const double *emf, const CP &src, const CP &u_stage,
+                                            const CP &u_base, double beta, double bdt,
+                                            const CP &u_out, double cs[Layout<MHD>::ncons]) {
+  constexpr int NC = Layout<MHD>::ncons;
+  const long n = b.ncell;
+  const long sj = b.ni, sk = (long)b.ni * b.nj;
+  const double a1 = b.dx[1] * b.dx[2], a2 = b.dx[0] * b.dx[2], a3 = b.dx[0] * b.dx[1];
+  const double vol = b.dx[0] * b.dx[1] * b.dx[2];
+  // every component is read and computed before anything is stored: U_s may be the same
+  // container as U^n (stage 1) and U_{s+1} the same as U^n (stage 2), so a store would
+  // keep the compiler from issuing the next component's loads ahead of it; with the
+  // stores last, all the loads of the update can be in flight at once.  (The geometric
+  // source terms exist exactly for the curved metrics.)
+  constexpr bool SRC = GEOM != PHX_GEOM_MINKOWSKI;
+  double usv[NC];
+  // with beta = 1 and U_s the same container as U^n (stage 1 of the RK2 cycle) the
+  // average 1 U_s + 0 U_s is U_s itself, bit for bit, for every finite or NaN component
+  // (an infinite one gives NaN): such a cell's U_s is not stored back
+  bool identity = beta == 1.0;
+#pragma unroll
+  for (int l = 0; l < NC; ++l) identity = identity && u_stage[l] == u_base[l];
+  bool inf_in = false;
+#pragma unroll
+  for (int l = 0; l < NC; ++l) {
+    double f[3][2];
+    face_fluxes<NDIM, CT && MHD>(flux, emf, l, c, n, sj, sk, f);
+    double du = a1 * f[0][1] - a1 * f[0][0];
+    if constexpr (NDIM >= 2) du += a2 * f[1][1] - a2 * f[1][0];
+    if constexpr (NDIM == 3) du += a3 * f[2][1] - a3 * f[2][0];
+    double dudt = ddiv(-du, vol);
+    if constexpr (SRC) {
+      if (l >= 1 && l <= 4) dudt = dudt + src[l][c];
+    }
+    const double us = u_stage[l][c];
+    usv[l] = beta * us + (1 - beta) * u_base[l][c];
+    inf_in = inf_in || isinf(us);
+    cs[l] = usv[l] + bdt * dudt;
+  }
+  if (!identity || inf_in) {
+#pragma unroll
+    for (int l = 0; l < NC; ++l) u_stage[l][c] = usv[l];
+  }
+  // U_{s+1} goes out before the inversion, which re-derives it only where it used a floor
+  // or ceiling (con2prim_fields); no conserved variable is live across the solve
+#pragma unroll
+  for (int l = 0; l < NC; ++l) u_out[l][c] = cs[l];
+}
+
 // interior cell t of block b: returns the cell's CFL time (DBL_MAX for t beyond the block
-// or when with_dt is false).  CT: take the magnetic fluxes from the corner EMFs in emf
-// (face_fluxes) instead of flux.
+// or when with_dt is false)
 template <bool MHD, int GEOM, bool CACHED = false, int NDIM = 3, bool CT = false, class FP,
           class CP, class PP>
 __device__ __forceinline__ double update_con2prim_body(
@@ -85,7 +139,6 @@ __device__ __forceinline__ double update_con2prim_body(
     double *__restrict__ mu, double *__restrict__ csig, const double *__restrict__ fsig,
     double *__restrict__ fail, int32_t *__restrict__ iters, bool with_dt,
     int c2p_mode = kC2pAll, const ColdQueue &cq = ColdQueue{}, int blk = 0) {
-  constexpr int NC = Layout<MHD>::ncons;
   const int ni = b.ie[0] - b.is[0] + 1, nj = b.ie[1] - b.is[1] + 1, nk = b.ie[2] - b.is[2] + 1;
   const bool active = t < (long)ni * nj * nk;
   double ldt_min = DBL_MAX;
@@ -96,48 +149,8 @@ __device__ __forceinline__ double update_con2prim_body(
     const long c = ((long)k * b.nj + j) * b.ni + i;
     const long n = b.ncell;
     const long sj = b.ni, sk = (long)b.ni * b.nj;
-    // parthenon FluxDivergence (uniform coordinates), SumData, AverageIndependentData,
-    // UpdateIndependentData -- the operation order of the separate kernels
-    const double a1 = b.dx[1] * b.dx[2], a2 = b.dx[0] * b.dx[2], a3 = b.dx[0] * b.dx[1];
-    const double vol = b.dx[0] * b.dx[1] * b.dx[2];
-    // every component is read and computed before anything is stored: U_s may be the same
-    // container as U^n (stage 1) and U_{s+1} the same as U^n (stage 2), so a store would
-    // keep the compiler from issuing the next component's loads ahead of it; with the
-    // stores last, all the loads of the update can be in flight at once.  (The geometric
-    // source terms exist exactly for the curved metrics.)
-    constexpr bool SRC = GEOM != PHX_GEOM_MINKOWSKI;
-    double cs[NC], usv[NC];
-    // with beta = 1 and U_s the same container as U^n (stage 1 of the RK2 cycle) the
-    // average 1 U_s + 0 U_s is U_s itself, bit for bit, for every finite or NaN component
-    // (an infinite one gives NaN): such a cell's U_s is not stored back
-    bool identity = beta == 1.0;
-#pragma unroll
-    for (int l = 0; l < NC; ++l) identity = identity && u_stage[l] == u_base[l];
-    bool inf_in = false;
-#pragma unroll
-    for (int l = 0; l < NC; ++l) {
-      double f[3][2];
-      face_fluxes<NDIM, CT && MHD>(flux, emf, l, c, n, sj, sk, f);
-      double du = a1 * f[0][1] - a1 * f[0][0];
-      if constexpr (NDIM >= 2) du += a2 * f[1][1] - a2 * f[1][0];
-      if constexpr (NDIM == 3) du += a3 * f[2][1] - a3 * f[2][0];
-      double dudt = ddiv(-du, vol);
-      if constexpr (SRC) {
-        if (l >= 1 && l <= 4) dudt = dudt + src[l][c];
-      }
-      const double us = u_stage[l][c];
-      usv[l] = beta * us + (1 - beta) * u_base[l][c];
-      inf_in = inf_in || isinf(us);
-      cs[l] = usv[l] + bdt * dudt;
-    }
-    if (!identity || inf_in) {
-#pragma unroll
-      for (int l = 0; l < NC; ++l) u_stage[l][c] = usv[l];
-    }
-    // U_{s+1} goes out before the inversion, which re-derives it only where it used a floor
-    // or ceiling (con2prim_fields); no conserved variable is live across the solve
-#pragma unroll
-    for (int l = 0; l < NC; ++l) u_out[l][c] = cs[l];
+    double cs[Layout<MHD>::ncons];
+    update_cell<MHD, GEOM, NDIM, CT>(b, c, flux, emf, src, u_stage, u_base, beta, bdt, u_out, cs);
     // kC2pWarm: a cell with no previous root to start from goes to the learned bracket
     if (c2p_mode == kC2pWarm && enqueue_cold(cq, !(mu[c] > 0.0), blk, c, false)) return DBL_MAX;
     // ConservedToPrimitive on U_{s+1}
@@ -196,6 +209,49 @@ __global__ __launch_bounds__(256) void k_update_con2prim(
     const double m = block_min(v);
     if (threadIdx.x == 0) partial[blockIdx.x] = m;
   }
+}
+
+// The update of the interior and the con2prim of the entire block on U_{s+1} (the ghosts from
+// what the container holds there): the one-block driver's stage up to its boundaries.
+template <bool MHD, int GEOM, int NDIM>
+__global__ __launch_bounds__(256) void k_update_con2prim_entire(
+    DevParams p, BlockGeom b, FluxPtrs flux, const double *__restrict__ emf, ConsPtrs src,
+    ConsPtrs u_stage, ConsPtrs u_base, double beta, double bdt, ConsPtrs u_out,
+    PrimPtrs prim_out, double *__restrict__ temp, double *__restrict__ mu,
+    double *__restrict__ csig, double *__restrict__ fail, int32_t *__restrict__ iters) {
+  constexpr int NC = Layout<MHD>::ncons;
+  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  int idx[3];
+  if (!entire_cell(b, c, idx)) return;
+  double cs[NC];
+  if (is_interior(b, idx)) {
+    update_cell<MHD, GEOM, NDIM, MHD && NDIM >= 2>(b, c, flux, emf, src, u_stage, u_base, beta,
+                                                   bdt, u_out, cs);
+  } else {
+#pragma unroll
+    for (int l = 0; l < NC; ++l) cs[l] = u_out[l][c];
+  }
+  con2prim_loaded<MHD, GEOM>(p, b, idx[0], idx[1], idx[2], cs, u_out, prim_out, temp, mu, csig,
+                             fail, iters);
+}
+
+void launch_update_con2prim_entire(const phx_fluid_params &p, const BlockGeom &bg, int ndim,
+                                   const FluxPtrs &flux, const double *emf, const ConsPtrs &src,
+                                   const ConsPtrs &u_stage, const ConsPtrs &u_base, double beta,
+                                   double dt, const ConsPtrs &u_out, const PrimPtrs &prim_out,
+                                   const phx_block_fields &f, int32_t *iters, hipStream_t s) {
+  with_geom(p.geom.kind, [&](auto G) {
+    with_mhd(p.mhd, [&](auto H) {
+      constexpr bool MH = decltype(H)::value;
+      constexpr int GM = decltype(G)::value;
+      auto kernel = ndim == 3   ? k_update_con2prim_entire<MH, GM, 3>
+                    : ndim == 2 ? k_update_con2prim_entire<MH, GM, 2>
+                                : k_update_con2prim_entire<MH, GM, 1>;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)((bg.ncell + 255) / 256)), dim3(256), 0, s,
+                         make_dev_params(&p), bg, flux, emf, src, u_stage, u_base, beta,
+                         beta * dt, u_out, prim_out, f.temp, f.c2p_mu, f.cell_sig, f.fail, iters);
+    });
+  });
 }
 
 // packs: the fused update over a work list of 3-D MHD blocks; dt from dt_dev when given

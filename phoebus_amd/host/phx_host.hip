@@ -16,35 +16,44 @@
 namespace phx {
 namespace host {
 
-template <class T>
-static bool dalloc(T **p, size_t n) {
-  if (hipMalloc(p, sizeof(T) * std::max<size_t>(n, 1)) != hipSuccess) return false;
-  return hipMemset(*p, 0, sizeof(T) * std::max<size_t>(n, 1)) == hipSuccess;
-}
-
 MeshBlockData::MeshBlockData(phx_ctx *ctx, const phx_fluid_params &p, const phx_block &b,
                              int ncontainers)
     : ctx_(ctx), p_(p), b_(b) {
   ncell_ = 1;
   for (int d = 0; d < 3; ++d) ncell_ *= b.nx[d] + (d < b.ndim ? 2 * b.ng : 0);
-  const long n = ncell_;
-  bool ok = true;
+  // one zeroed allocation, every field on a 256-byte boundary
+  const size_t n = ncell_, nc = ncons();
   cons_.assign(ncontainers, nullptr);
-  for (auto &c : cons_) ok = ok && dalloc(&c, ncons() * n);
-  ok = ok && dalloc(&f_.prim, nprim() * n) && dalloc(&f_.temp, n) && dalloc(&f_.c2p_mu, n) &&
-       dalloc(&f_.fail, n) && dalloc(&f_.cell_sig, 3 * n) && dalloc(&f_.face_sig, 3 * n) &&
-       dalloc(&f_.flux, 3 * ncons() * n) && dalloc(&f_.emf, 3 * n) &&
-       dalloc(&f_.src, ncons() * n) && dalloc(&f_.iters, n) && dalloc(&f_.dt, 1);
-  ok_ = ok;
+  struct Field {
+    double **q;
+    size_t count;
+  };
+  double *iters = nullptr;
+  std::vector<Field> fields;
+  for (auto &c : cons_) fields.push_back({&c, nc * n});
+  for (const Field &x : {Field{&f_.prim, nprim() * n}, Field{&f_.temp, n}, Field{&f_.c2p_mu, n},
+                         Field{&f_.fail, n}, Field{&f_.cell_sig, 3 * n},
+                         Field{&f_.face_sig, 3 * n}, Field{&f_.flux, 3 * nc * n},
+                         Field{&f_.emf, 3 * n}, Field{&f_.src, nc * n},
+                         Field{&iters, (n + 1) / 2}})
+    fields.push_back(x);
+  size_t total = 0;
+  for (const Field &x : fields) total += (x.count + 31) / 32 * 32;
+  ok_ = hipMalloc(&arena_, sizeof(double) * total) == hipSuccess &&
+        hipMemset(arena_, 0, sizeof(double) * total) == hipSuccess &&
+        hipHostMalloc(&f_.dt, sizeof(double), hipHostMallocDefault) == hipSuccess;
+  if (!ok_) return;
+  double *q = arena_;
+  for (const Field &x : fields) {
+    *x.q = q;
+    q += (x.count + 31) / 32 * 32;
+  }
+  f_.iters = reinterpret_cast<int32_t *>(iters);
 }
 
 MeshBlockData::~MeshBlockData() {
-  for (auto c : cons_)
-    if (c) (void)hipFree(c);
-  for (void *q : {(void *)f_.prim, (void *)f_.temp, (void *)f_.c2p_mu, (void *)f_.fail,
-                  (void *)f_.cell_sig, (void *)f_.face_sig, (void *)f_.flux, (void *)f_.emf,
-                  (void *)f_.src, (void *)f_.iters, (void *)f_.dt})
-    if (q) (void)hipFree(q);
+  if (arena_) (void)hipFree(arena_);
+  if (f_.dt) (void)hipHostFree(f_.dt);
 }
 
 phx_block_fields MeshBlockData::fields(int container) const {
@@ -106,14 +115,14 @@ TaskStatus ConservedToPrimitive(MeshBlockData *rc, int container) {
 }
 double EstimateTimestepBlock(MeshBlockData *rc, bool &has_face_speeds, double cfl) {
   const phx_block_fields f = rc->fields(0);
-  double h = -1.0;
+  // the reduction writes the host's scalar itself: a copy after it was a launch and a second
+  // wait, 10 us of a 512-cell block's cycle
   const bool ok =
       phx_estimate_dt(rc->ctx(), &rc->params(), &rc->block(), &f, has_face_speeds ? 1 : 0, cfl,
                       rc->shared().dt, nullptr) == PHX_OK &&
-      hipStreamSynchronize(rc->ctx()->stream) == hipSuccess &&
-      hipMemcpy(&h, rc->shared().dt, sizeof(double), hipMemcpyDeviceToHost) == hipSuccess;
+      hipStreamSynchronize(rc->ctx()->stream) == hipSuccess;
   has_face_speeds = true;  // fluid.cpp:940
-  return ok ? h : -1.0;
+  return ok ? *static_cast<volatile double *>(rc->shared().dt) : -1.0;
 }
 }  // namespace fluid
 
@@ -139,15 +148,40 @@ TaskStatus FluxDivergenceUpdate(MeshBlockData *rc, int stage_container, int base
                                        rc->cons(stage_container), rc->cons(base_container),
                                        beta, dt, rc->cons(out_container), nullptr));
 }
+
+// A small block's stage is a chain of launches of 3 to 8 us each; the update (4.9 us at 512
+// cells) and its gap go into the con2prim's launch, which the bits do not show: a cell's
+// con2prim reads its own U_{s+1} alone.
+TaskStatus UpdateFillDerived(MeshBlockData *rc, int stage_container, int base_container,
+                             double beta, double dt, int out_container) {
+  const phx_block_fields f = rc->fields(0);
+  const phx_block &b = rc->block();
+  const BlockGeom bg = make_block_geom(&b);
+  const int nc = rc->ncons(), np = rc->nprim();
+  hipStream_t s = rc->ctx()->stream;
+  const FluxPtrs flux = flux_ptrs(&f, bg.ncell, nc);
+  if (rc->params().mhd && b.ndim > 1) {
+    if (b.ng < 2) return TaskStatus::fail;
+    launch_ct_emf(bg, flux, f.emf, s);
+  }
+  const bool curved = rc->params().geom.kind != PHX_GEOM_MINKOWSKI;
+  launch_update_con2prim_entire(
+      rc->params(), bg, b.ndim, flux, f.emf, ConsPtrs::contiguous(curved ? f.src : nullptr, curved ? bg.ncell : 0),
+      ConsPtrs::contiguous(rc->cons(stage_container), bg.ncell),
+      ConsPtrs::contiguous(rc->cons(base_container), bg.ncell), beta, dt,
+      ConsPtrs::contiguous(rc->cons(out_container), bg.ncell), prim_ptrs(&f, bg.ncell, np), f,
+      rc->shared().iters, s);
+  return hipGetLastError() == hipSuccess ? TaskStatus::complete : TaskStatus::fail;
+}
 }  // namespace update
 
 namespace boundaries {
 
-// fills the ghost layers of dimension d on one side; outflow copies the first interior
+// fills the ghost layers of dimension d on both sides; outflow copies the first interior
 // layer scaled by sqrt(gamma)(ghost) / sqrt(gamma)(ref), periodic copies the opposite
-// interior layers
+// interior layers (neither side reads the other's ghosts, so both are one launch)
 template <int GEOM>
-__global__ void k_bc(BlockGeom b, DevParams p, int d, int side, int periodic, int nv,
+__global__ void k_bc(BlockGeom b, DevParams p, int d, int periodic0, int periodic1, int nv,
                      double *__restrict__ q) {
   using M = typename MetricOf<GEOM>::type;
   const int n[3] = {b.ni, b.nj, b.nk};
@@ -156,8 +190,11 @@ __global__ void k_bc(BlockGeom b, DevParams p, int d, int side, int periodic, in
   const long span1 = d == 1 ? ng : n[1];
   const long span2 = d == 2 ? ng : n[2];
   const long total = span0 * span1 * span2;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= total) return;
+  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 2 * total) return;
+  const int side = t >= total;
+  t -= side ? total : 0;
+  const int periodic = side ? periodic1 : periodic0;
   int idx[3] = {(int)(t % span0), (int)((t / span0) % span1), (int)(t / (span0 * span1))};
   if (side == 1) idx[d] += b.ie[d] + 1;  // outer ghosts
   int ref[3] = {idx[0], idx[1], idx[2]};
@@ -173,7 +210,13 @@ __global__ void k_bc(BlockGeom b, DevParams p, int d, int side, int periodic, in
     const M gr(p, xc(b, 0, ref[0]), xc(b, 1, ref[1]), xc(b, 2, ref[2]));
     gratio = ratio(g.detgamma(), gr.detgamma());
   }
-  for (int l = 0; l < nv; ++l) q[l * b.ncell + c] = gratio * q[l * b.ncell + cr];
+  double u[8];  // all read before any is written: one memory round trip
+#pragma unroll
+  for (int l = 0; l < 8; ++l)
+    if (l < nv) u[l] = q[l * b.ncell + cr];
+#pragma unroll
+  for (int l = 0; l < 8; ++l)
+    if (l < nv) q[l * b.ncell + c] = gratio * u[l];
 }
 
 TaskStatus ApplyBoundaryConditions(MeshBlockData *rc, int container, const Kind kinds[6]) {
@@ -182,16 +225,14 @@ TaskStatus ApplyBoundaryConditions(MeshBlockData *rc, int container, const Kind 
   hipStream_t s = rc->ctx()->stream;
   for (int d = 0; d < rc->block().ndim; ++d) {
     const int n[3] = {bg.ni, bg.nj, bg.nk};
-    long total = 1;
+    long total = 2;
     for (int e = 0; e < 3; ++e) total *= e == d ? bg.ng : n[e];
-    for (int side = 0; side < 2; ++side) {
-      const int periodic = kinds[2 * d + side] == Kind::periodic;
-      const unsigned blocks = (unsigned)((total + 255) / 256);
-      with_geom(rc->params().geom.kind, [&](auto G) {
-        hipLaunchKernelGGL((k_bc<decltype(G)::value>), dim3(blocks), dim3(256), 0, s, bg, dp, d,
-                           side, periodic, rc->ncons(), rc->cons(container));
-      });
-    }
+    const unsigned blocks = (unsigned)((total + 255) / 256);
+    with_geom(rc->params().geom.kind, [&](auto G) {
+      hipLaunchKernelGGL((k_bc<decltype(G)::value>), dim3(blocks), dim3(256), 0, s, bg, dp, d,
+                         kinds[2 * d] == Kind::periodic, kinds[2 * d + 1] == Kind::periodic,
+                         rc->ncons(), rc->cons(container));
+    });
   }
   return hipGetLastError() == hipSuccess ? TaskStatus::complete : TaskStatus::fail;
 }
@@ -208,6 +249,10 @@ Driver::Driver(MeshBlockData *rc, const boundaries::Kind kinds[6], double cfl,
 
 TaskStatus Driver::FillDerived(int container) {
   if (fluid::ConservedToPrimitive(rc_, container) != TaskStatus::complete) return TaskStatus::fail;
+  return Fixups(container);
+}
+
+TaskStatus Driver::Fixups(int container) {
   if (fixup::ConservedToPrimitiveFixup(rc_, container, fx_) != TaskStatus::complete)
     return TaskStatus::fail;
   return fixup::ApplyFloors(rc_, container, fx_);
@@ -240,11 +285,10 @@ TaskStatus Driver::RungeKuttaStage(int stage) {
   if (curved && fluid::CalculateFluidSourceTerms(rc_) != TaskStatus::complete)
     return TaskStatus::fail;
   if (fluid::CalculateFluxes(rc_) != TaskStatus::complete) return TaskStatus::fail;
-  if (fluid::FluxCT(rc_) != TaskStatus::complete) return TaskStatus::fail;
-  if (update::FluxDivergenceUpdate(rc_, sc0, kBase, beta[stage - 1], dt_, sc1) !=
+  if (update::UpdateFillDerived(rc_, sc0, kBase, beta[stage - 1], dt_, sc1) !=
       TaskStatus::complete)
     return TaskStatus::fail;
-  if (FillDerived(sc1) != TaskStatus::complete) return TaskStatus::fail;
+  if (Fixups(sc1) != TaskStatus::complete) return TaskStatus::fail;
   if (boundaries::ApplyBoundaryConditions(rc_, sc1, kinds_) != TaskStatus::complete)
     return TaskStatus::fail;
   return FillDerived(sc1);

@@ -28,7 +28,7 @@ struct BlockFields {
   double *cell_sig = nullptr, *face_sig = nullptr, *flux = nullptr, *emf = nullptr;
   double *src = nullptr;
   int32_t *iters = nullptr;
-  double *dt = nullptr;  // one device scalar for the timestep reduction
+  double *dt = nullptr;  // the timestep reduction's scalar, in pinned host memory
 };
 
 class MeshBlockData {
@@ -58,6 +58,7 @@ class MeshBlockData {
   phx_fluid_params p_;
   phx_block b_;
   long ncell_ = 0;
+  double *arena_ = nullptr;  // every device field
   std::vector<double *> cons_;
   BlockFields f_;
   bool ok_ = false;
@@ -90,6 +91,10 @@ namespace update {
 // phoebus_driver.cpp:560-576: containers by index
 TaskStatus FluxDivergenceUpdate(MeshBlockData *rc, int stage_container, int base_container,
                                 double beta, double dt, int out_container);
+// fluid::FluxCT (its corner EMFs; the shared flux field keeps the Riemann solver's magnetic
+// fluxes), FluxDivergenceUpdate and fluid::ConservedToPrimitive of the out container
+TaskStatus UpdateFillDerived(MeshBlockData *rc, int stage_container, int base_container,
+                             double beta, double dt, int out_container);
 }  // namespace update
 
 namespace boundaries {
@@ -131,6 +136,8 @@ class Driver {
   phx_fixup_params fx_ = {0, PHX_FAILURE_INTERPOLATE, 0, 0, 50.0, 2500.0};
   // FillDerived on one container followed by the fixup tasks
   TaskStatus FillDerived(int container);
+  // the fixup tasks alone
+  TaskStatus Fixups(int container);
 };
 
 }  // namespace host

@@ -657,6 +657,41 @@ def test_one_launch_sweeps_match_separate(phx, nx, recon, mhd):
     assert not np.all(got[0][0] == 7.5)
 
 
+@pytest.mark.parametrize("nx", [(1,), (2048,), (2049,), (45, 45), (46, 45), (12, 13, 13),
+                                (13, 13, 13)])
+@pytest.mark.parametrize("face", [False, True])
+def test_estimate_dt_one_and_many_groups(phx, nx, face):
+    """The CFL time of blocks on both sides of the size that one workgroup takes: the bits of
+    the cell-wise formula, wherever the least time is."""
+    say(f"[gpu] estimate_dt {nx} face speeds {face}")
+    rng = np.random.default_rng(nx[0] + len(nx))
+    nd, ng = len(nx), 4
+    b = block(nd, nx, ng, dx=(0.1, 0.2, 0.3))
+    p = fluid_params(gamma=1.4, mhd=False)
+    st = BlockState(p, b)
+    out = DeviceArray((1,))
+    inner = tuple(slice(ng, ng + n) for n in nx[::-1])
+    inner = (0,) * (3 - nd) + inner if nd < 3 else inner
+    for fast in (0, -1, None):
+        cs = rng.uniform(0.1, 0.9, st.cell_sig.shape)
+        fs = rng.uniform(0.1, 0.9, st.face_sig.shape)
+        if fast is not None:  # the first or the last cell decides
+            cs[(0,) + inner][(fast,) * nd] = 7.0
+        st.cell_sig.upload(cs)
+        st.face_sig.upload(fs)
+        phx.estimate_dt(p, b, st.fields(), face, 0.3, out)
+        synchronize()
+        ldt = 0.0
+        for d in range(nd):
+            s = cs[d][inner]
+            if face:
+                up = list(inner)
+                up[2 - d] = slice(ng + 1, ng + 1 + nx[d])
+                s = np.maximum(s, np.maximum(fs[d][inner], fs[d][tuple(up)]))
+            ldt = ldt + s / b.dx[d]
+        assert out.get()[0] == 0.3 * np.min(1.0 / (ldt + 1e-50))
+
+
 @pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
 @pytest.mark.parametrize("nx,mhd", [((64, 64, 33), True), ((72, 72, 51), True),
                                     ((72, 72, 50), False)])
