@@ -143,7 +143,9 @@ int check_block(phx_ctx *ctx, const phx_block *b, int recon);
 
 void launch_flux_ct(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s);
 // FluxCT's corner EMFs alone (the fused updates form the rewritten B fluxes from them)
-void launch_ct_emf(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s);
+// the corner EMFs; dt given: also dt[0] = dt0, for kernels after it that lower it
+void launch_ct_emf(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s,
+                   double *dt = nullptr, double dt0 = 0.0);
 // the update of the interior (beta, dt as in phx_flux_divergence_update; with MHD in 2-D and 3-D
 // the magnetic fluxes from the corner EMFs) and the con2prim of the entire block on u_out
 void launch_update_con2prim_entire(const phx_fluid_params &p, const BlockGeom &bg, int ndim,

@@ -41,7 +41,9 @@ __device__ __forceinline__ void ct_emf_3d_body(const BlockGeom &b, long t, const
 
 template <int NC>
 __global__ __launch_bounds__(256) void k_ct_emf_3d(BlockGeom b, FluxPtrs flux,
-                                                   double *__restrict__ emf) {
+                                                   double *__restrict__ emf,
+                                                   double *__restrict__ dt, double dt0) {
+  if (dt && blockIdx.x == 0 && threadIdx.x == 0) dt[0] = dt0;
   ct_emf_3d_body<NC>(b, (long)blockIdx.x * blockDim.x + threadIdx.x, flux, emf);
 }
 
@@ -77,7 +79,9 @@ __global__ __launch_bounds__(256) void k_ct_flux_3d(BlockGeom b, FluxPtrs flux,
 
 template <int NC>
 __global__ __launch_bounds__(256) void k_ct_emf_2d(BlockGeom b, FluxPtrs flux,
-                                                   double *__restrict__ emf) {
+                                                   double *__restrict__ emf,
+                                                   double *__restrict__ dt, double dt0) {
+  if (dt && blockIdx.x == 0 && threadIdx.x == 0) dt[0] = dt0;
   const int ni = b.ie[0] - b.is[0] + 2, nj = b.ie[1] - b.is[1] + 2, nk = b.ie[2] - b.is[2] + 1;
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)ni * nj * nk) return;
@@ -734,15 +738,18 @@ void launch_pack_ct_emf(const PackView &v, long groups, hipStream_t s) {
   hipLaunchKernelGGL(k_pack_ct_emf<8>, dim3((unsigned)groups), dim3(256), 0, s, v);
 }
 
-void launch_ct_emf(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s) {
+void launch_ct_emf(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s,
+                   double *dt, double dt0) {
   const int nx0 = bg.ie[0] - bg.is[0] + 1, nx1 = bg.ie[1] - bg.is[1] + 1;
   const int nx2 = bg.ie[2] - bg.is[2] + 1;
   if (bg.ndim == 3) {
     const long n = (long)(nx0 + 1) * (nx1 + 1) * (nx2 + 1);
-    hipLaunchKernelGGL(k_ct_emf_3d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf);
+    hipLaunchKernelGGL(k_ct_emf_3d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf,
+                       dt, dt0);
   } else {
     const long n = (long)(nx0 + 1) * (nx1 + 1) * nx2;
-    hipLaunchKernelGGL(k_ct_emf_2d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf);
+    hipLaunchKernelGGL(k_ct_emf_2d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf,
+                       dt, dt0);
   }
 }
 
@@ -751,11 +758,13 @@ void launch_flux_ct(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipS
   const int nx2 = bg.ie[2] - bg.is[2] + 1;
   if (bg.ndim == 3) {
     const long n = (long)(nx0 + 1) * (nx1 + 1) * (nx2 + 1);
-    hipLaunchKernelGGL(k_ct_emf_3d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf);
+    hipLaunchKernelGGL(k_ct_emf_3d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf,
+                       nullptr, 0.0);
     hipLaunchKernelGGL(k_ct_flux_3d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf);
   } else {
     const long n = (long)(nx0 + 1) * (nx1 + 1) * nx2;
-    hipLaunchKernelGGL(k_ct_emf_2d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf);
+    hipLaunchKernelGGL(k_ct_emf_2d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf,
+                       nullptr, 0.0);
     hipLaunchKernelGGL(k_ct_flux_2d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf);
   }
 }

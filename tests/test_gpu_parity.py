@@ -692,6 +692,38 @@ def test_estimate_dt_one_and_many_groups(phx, nx, face):
         assert out.get()[0] == 0.3 * np.min(1.0 / (ldt + 1e-50))
 
 
+@pytest.mark.parametrize("nx,mhd", [((4, 4), True), ((16, 16), True), ((33, 31, 8), True),
+                                    ((40, 30), False), ((300,), True)])
+@pytest.mark.parametrize("cfl", [0.4, 0.0])
+def test_stage_dt_is_that_of_its_speeds(phx, nx, mhd, cfl):
+    """The stage's CFL time (found in the update, or by the finishing launch without CT or with
+    cfl = 0) is phx_estimate_dt of the speeds it leaves, call after call as it rises and falls."""
+    say(f"[gpu] stage dt {nx} mhd {mhd} cfl {cfl}")
+    rng = np.random.default_rng(sum(nx))
+    b = geom_block(len(nx), nx, A.GEOM_MINKOWSKI)
+    p = fluid_params(gamma=4 / 3, mhd=mhd, recon=A.RECON_WENO5Z, riemann=A.RIEMANN_HLL,
+                     c2p_tol=1e-10)
+    st = BlockState(p, b)
+    u_out, prim_out = DeviceArray(st.cons.shape), DeviceArray(st.prim.shape)
+    out, want = DeviceArray((1,)), DeviceArray((1,))
+    prim = random_block(rng, b, mhd, 4 / 3, A.GEOM_MINKOWSKI)
+    got = []
+    for scale in (1.0, 0.05, 1.0):
+        q = prim.copy()
+        q[1:4] *= scale
+        q[4] *= scale
+        q[(8 if mhd else 5)] *= scale
+        st.prim.upload(q)
+        phx.prim_to_con(p, b, st.fields())
+        phx.fluid_stage(p, b, st.fields(), 1.0, 1e-4, st.cons, u_out, prim_out, cfl=cfl,
+                        dt_out=out)
+        phx.estimate_dt(p, b, st.fields(), True, cfl, want)
+        synchronize()
+        assert out.get()[0] == want.get()[0]
+        got.append(out.get()[0])
+    assert got[0] == got[2] and (cfl == 0.0 or got[1] != got[0])  # one rise, one fall
+
+
 @pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
 @pytest.mark.parametrize("nx,mhd", [((64, 64, 33), True), ((72, 72, 51), True),
                                     ((72, 72, 50), False)])
