@@ -146,6 +146,10 @@ void launch_flux_ct(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipS
 // the corner EMFs; dt given: also dt[0] = dt0, for kernels after it that lower it
 void launch_ct_emf(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s,
                    double *dt = nullptr, double dt0 = 0.0);
+// the corner EMFs and the sources of a curved MHD block (2-D, 3-D) in one launch
+void launch_sources_emf(int geom, const DevParams &dp, const BlockGeom &bg, const PrimPtrs &prim,
+                        const ConsPtrs &src, const FluxPtrs &flux, double *emf, hipStream_t s,
+                        double *dt = nullptr, double dt0 = 0.0);
 // the update of the interior (beta, dt as in phx_flux_divergence_update; with MHD in 2-D and 3-D
 // the magnetic fluxes from the corner EMFs) and the con2prim of the entire block on u_out
 void launch_update_con2prim_entire(const phx_fluid_params &p, const BlockGeom &bg, int ndim,

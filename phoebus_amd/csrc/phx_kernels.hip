@@ -77,13 +77,9 @@ __global__ __launch_bounds__(256) void k_ct_flux_3d(BlockGeom b, FluxPtrs flux,
   ct_flux_3d_body<NC>(b, (long)blockIdx.x * blockDim.x + threadIdx.x, flux, emf);
 }
 
-template <int NC>
-__global__ __launch_bounds__(256) void k_ct_emf_2d(BlockGeom b, FluxPtrs flux,
-                                                   double *__restrict__ emf,
-                                                   double *__restrict__ dt, double dt0) {
-  if (dt && blockIdx.x == 0 && threadIdx.x == 0) dt[0] = dt0;
+__device__ __forceinline__ void ct_emf_2d_body(const BlockGeom &b, long t, const FluxPtrs &flux,
+                                               double *__restrict__ emf) {
   const int ni = b.ie[0] - b.is[0] + 2, nj = b.ie[1] - b.is[1] + 2, nk = b.ie[2] - b.is[2] + 1;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)ni * nj * nk) return;
   const int i = (int)(t % ni) + b.is[0];
   const int j = (int)((t / ni) % nj) + b.is[1];
@@ -92,6 +88,14 @@ __global__ __launch_bounds__(256) void k_ct_emf_2d(BlockGeom b, FluxPtrs flux,
   const long sj = b.ni;
   auto F = [&](int d, int comp, long cc) { return flux[d * 8 + 5 + comp][cc]; };
   emf[c] = 0.25 * (F(0, 1, c) + F(0, 1, c - sj) - F(1, 0, c) - F(1, 0, c - 1));
+}
+
+template <int NC>
+__global__ __launch_bounds__(256) void k_ct_emf_2d(BlockGeom b, FluxPtrs flux,
+                                                   double *__restrict__ emf,
+                                                   double *__restrict__ dt, double dt0) {
+  if (dt && blockIdx.x == 0 && threadIdx.x == 0) dt[0] = dt0;
+  ct_emf_2d_body(b, (long)blockIdx.x * blockDim.x + threadIdx.x, flux, emf);
 }
 
 template <int NC>
@@ -518,6 +522,28 @@ __global__ __launch_bounds__(128) void k_sources(DevParams p, BlockGeom b, int k
   sources_body<MHD, GEOM>(p, b, (long)blockIdx.x * blockDim.x + threadIdx.x, kb, prim, src);
 }
 
+// Sources and corner EMFs in one launch: the first ns groups take the sources, whose lanes run
+// longest, the others the EMFs.  The sources wait on the metric's serial chain, the EMFs on
+// memory; neither fills the chip.  us, one launch against two: FMKS 16^3 16.9 / 23.2, 64x64x32
+// 29.0 / 34.7, 72^3 36.7 / 47.1, 96^3 69.6 / 82.2; Kerr-Schild 256x128 7.8 / 14.0, 64^3 17.5 /
+// 23.1, 96^3 38.3 / 48.9.
+template <int GEOM, int NDIM>
+__global__ __launch_bounds__(128) void k_sources_emf(DevParams p, BlockGeom b, int kb, unsigned ns,
+                                                     PrimPtrs prim, ConsPtrs src, FluxPtrs flux,
+                                                     double *__restrict__ emf,
+                                                     double *__restrict__ dt, double dt0) {
+  if (blockIdx.x < ns) {
+    sources_body<true, GEOM>(p, b, (long)blockIdx.x * 128 + threadIdx.x, kb, prim, src);
+    return;
+  }
+  const unsigned g = blockIdx.x - ns;
+  if (dt && g == 0 && threadIdx.x == 0) dt[0] = dt0;
+  if constexpr (NDIM == 3)
+    ct_emf_3d_body<8>(b, (long)g * 128 + threadIdx.x, flux, emf);
+  else
+    ct_emf_2d_body(b, (long)g * 128 + threadIdx.x, flux, emf);
+}
+
 template <int NC>
 __global__ void k_zero_sources(BlockGeom b, ConsPtrs src) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -767,6 +793,25 @@ void launch_flux_ct(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipS
                        nullptr, 0.0);
     hipLaunchKernelGGL(k_ct_flux_2d<8>, dim3(nblocks(n, 256)), dim3(256), 0, s, bg, flux, emf);
   }
+}
+
+void launch_sources_emf(int geom, const DevParams &dp, const BlockGeom &bg, const PrimPtrs &prim,
+                        const ConsPtrs &src, const FluxPtrs &flux, double *emf, hipStream_t s,
+                        double *dt, double dt0) {
+  const int nx0 = bg.ie[0] - bg.is[0] + 1, nx1 = bg.ie[1] - bg.is[1] + 1;
+  const int nk = bg.ie[2] - bg.is[2] + 1;
+  const long cols = (long)nx0 * nx1;
+  const int kb = source_cells(cols * nk);
+  const unsigned ns = nblocks(cols * ((nk + kb - 1) / kb), 128);
+  const unsigned ne = nblocks((long)(nx0 + 1) * (nx1 + 1) * (bg.ndim == 3 ? nk + 1 : nk), 128);
+  with_geom(geom, [&](auto G) {
+    constexpr int GEOM = decltype(G)::value;
+    if constexpr (GEOM != PHX_GEOM_MINKOWSKI) {
+      auto kernel = bg.ndim == 3 ? k_sources_emf<GEOM, 3> : k_sources_emf<GEOM, 2>;
+      hipLaunchKernelGGL(kernel, dim3(ns + ne), dim3(128), 0, s, dp, bg, kb, ns, prim, src, flux,
+                         emf, dt, dt0);
+    }
+  });
 }
 
 void launch_sources(int geom, int mhd, const DevParams &dp, const BlockGeom &bg,

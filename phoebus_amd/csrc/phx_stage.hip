@@ -407,12 +407,17 @@ static int fluid_stage_launches(phx_ctx *ctx, const phx_fluid_params *p, const p
   }
   const bool ct = p->mhd && b->ndim > 1;
   const bool dt_direct = a->dt_out && ct && a->cfl > 0.0;
-  if (ct) {  // FluxCT: the EMFs here, the B-flux rewrite in the update
-    ctx->mark_begin("flux_ct", s);
-    launch_ct_emf(bg, flux, f->emf, s, dt_direct ? a->dt_out : nullptr, a->cfl * DBL_MAX);
+  // FluxCT: the EMFs here, the B-flux rewrite in the update
+  double *dt = dt_direct ? a->dt_out : nullptr;
+  if (ct && curved) {
+    ctx->mark_begin("sources_ct", s);
+    launch_sources_emf(p->geom.kind, dp, bg, prim, src_c, flux, f->emf, s, dt, a->cfl * DBL_MAX);
     ctx->mark_end(s);
-  }
-  if (curved) {
+  } else if (ct) {
+    ctx->mark_begin("flux_ct", s);
+    launch_ct_emf(bg, flux, f->emf, s, dt, a->cfl * DBL_MAX);
+    ctx->mark_end(s);
+  } else if (curved) {
     ctx->mark_begin("sources", s);
     launch_sources(p->geom.kind, p->mhd, dp, bg, prim, src_c, s);
     ctx->mark_end(s);
@@ -423,7 +428,7 @@ static int fluid_stage_launches(phx_ctx *ctx, const phx_fluid_params *p, const p
   ctx->mark_begin("update_con2prim", s);
 #define ARGS dp, bg, flux, f->emf, src, cons, u_base, a->beta, bdt, u_out, prim_out, \
              f->temp, f->c2p_mu, f->cell_sig, f->face_sig, f->fail, a->iters, partial, \
-             dt_direct ? a->dt_out : nullptr, a->cfl
+             dt, a->cfl
   with_geom(p->geom.kind, [&](auto G) {
     with_mhd(p->mhd, [&](auto H) {
       constexpr bool MH = decltype(H)::value;

@@ -725,6 +725,31 @@ def test_stage_dt_is_that_of_its_speeds(phx, nx, mhd, cfl):
 
 
 @pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
+@pytest.mark.parametrize("nx", [(4, 4), (31, 17), (127, 1, 1), (16, 8, 16), (52, 51, 53)])
+def test_stage_sources_with_emfs_match_the_tasks(phx, geom, nx):
+    """A curved MHD stage's sources and corner EMFs, one launch, are those of the two tasks."""
+    say(f"[gpu] sources and EMFs in one launch geom {geom} {nx}")
+    b = geom_block(len(nx), nx, geom)
+    p = geom_params(geom, gamma=13.0 / 9.0, mhd=True, recon=A.RECON_WENO5Z,
+                    riemann=A.RIEMANN_HLL)
+    prim = random_block(np.random.default_rng(sum(nx)), b, True, 13.0 / 9.0, geom)
+    st, ref = BlockState(p, b), BlockState(p, b)
+    for x in (st, ref):
+        x.prim.upload(prim)
+        phx.prim_to_con(p, b, x.fields())
+    u_out, prim_out = DeviceArray(st.cons.shape), DeviceArray(st.prim.shape)
+    phx.fluid_stage(p, b, st.fields(with_src=True), 1.0, 1e-4, st.cons, u_out, prim_out,
+                    dt_out=DeviceArray((1,)))
+    f = ref.fields(with_src=True)
+    phx.calculate_fluxes(p, b, f)
+    phx.flux_ct(p, b, f)
+    phx.fluid_source_terms(p, b, f)
+    synchronize()
+    np.testing.assert_array_equal(st.emf.get(), ref.emf.get())
+    np.testing.assert_array_equal(st.src.get(), ref.src.get())
+
+
+@pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
 @pytest.mark.parametrize("nx,mhd", [((64, 64, 33), True), ((72, 72, 51), True),
                                     ((72, 72, 50), False)])
 def test_sources_of_several_cells_per_lane(phx, geom, nx, mhd):
