@@ -211,8 +211,8 @@ void launch_pack_flux(int d, int recon, int riemann, int geom, const DevParams &
                       const PackView &v, long groups, TileShape sh, hipStream_t s);
 }  // namespace flux_fast
 void launch_pack_ct_emf(const PackView &v, long groups, hipStream_t s);
-void launch_pack_sources(int geom, const DevParams &dp, const PackView &v, long groups, int kb,
-                         hipStream_t s);
+void launch_pack_sources_emf(int geom, const DevParams &dp, const PackView &vs, long groups_s,
+                             int kb, const PackView &ve, long groups_e, hipStream_t s);
 // The cells a plain con2prim pass leaves to the learned bracket: those with no previous
 // root (mu <= 0: initial data, fresh cells).  Entries are (block << 32) | (keep << 31) |
 // cell, keep = 1 for a cell whose iteration count is not to be written (an interior cell

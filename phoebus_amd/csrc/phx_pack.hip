@@ -90,15 +90,15 @@ void launch_stage_fluxes(phx_ctx *ctx, phx_pack *k, int st, hipStream_t s) {
     ctx->mark_end(s);
   }
   // FluxCT: the corner EMFs here; the update forms the rewritten B fluxes from them
-  ctx->mark_begin("flux_ct", s);
-  launch_pack_ct_emf(view(k, st, 3), k->groups[3], s);
-  ctx->mark_end(s);
   if (k->p.geom.kind != PHX_GEOM_MINKOWSKI) {
-    ctx->mark_begin("sources", s);
-    launch_pack_sources(k->p.geom.kind, k->dp, view(k, st, 8), k->groups[8], k->src_cells,
-                        s);
-    ctx->mark_end(s);
+    ctx->mark_begin("sources_ct", s);
+    launch_pack_sources_emf(k->p.geom.kind, k->dp, view(k, st, 8), k->groups[8], k->src_cells,
+                            view(k, st, 3), k->groups[3], s);
+  } else {
+    ctx->mark_begin("flux_ct", s);
+    launch_pack_ct_emf(view(k, st, 3), k->groups[3], s);
   }
+  ctx->mark_end(s);
 }
 
 void launch_stage(phx_ctx *ctx, phx_pack *k, const phx_pack_stage_args *a, hipStream_t s) {
