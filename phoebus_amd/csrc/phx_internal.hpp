@@ -252,6 +252,11 @@ void launch_pack_update(int geom, const DevParams &dp, const PackView &v, long g
                         double beta, double dt, const double *dt_dev, double *partial,
                         hipStream_t s, int c2p_mode = kC2pAll, const ColdQueue &cq = ColdQueue{},
                         double *extra = nullptr);
+// the same without dt reduction and learned bracket, with the con2prim of the face-adjacent ghost
+// layer (work list vf) on the stage's output in the same launch
+void launch_pack_update_with_faces(int geom, const DevParams &dp, const PackView &v, long groups,
+                                   const PackView &vf, long groups_f, double beta, double dt,
+                                   hipStream_t s);
 // con2prim with the learned bracket over the queued cells of a pack (phx_mlp.hip), in a
 // grid-stride loop over the count the producing pass left; counters (nullable)
 // accumulate [bracket misses, network-bracketed solves]; extra (nullable, interior cells

@@ -305,15 +305,22 @@ int run_stage(phx_mesh *m, int st, bool last, hipStream_t s) {
     ctx->mark_end(s);
   }
   const bool learned = k->mlp != nullptr;
-  ctx->mark_begin(learned ? "update" : "update_con2prim", s);
-  launch_pack_update(k->p.geom.kind, k->dp, pv(m, st, 4), k->groups[4], st == 1 ? 1.0 : 0.5,
-                     m->dt, nullptr, nullptr, s, learned ? kC2pWarm : kC2pAll, k->cq);
-  ctx->mark_end(s);
+  const double beta = st == 1 ? 1.0 : 0.5;
   // the first FillDerived: the interior (inverted by the update) and the face-adjacent
   // ghost layer the fixup reads; with the learned bracket, the cells of both with no
   // previous root go through one learned pass
-  launch_c2p(m, st, 6, s, learned);
-  if (learned) launch_c2p_queued(m, st, "con2prim_learned_first", s);
+  ctx->mark_begin(learned ? "update" : "update_con2prim", s);
+  if (learned)
+    launch_pack_update(k->p.geom.kind, k->dp, pv(m, st, 4), k->groups[4], beta, m->dt, nullptr,
+                       nullptr, s, kC2pWarm, k->cq);
+  else
+    launch_pack_update_with_faces(k->p.geom.kind, k->dp, pv(m, st, 4), k->groups[4],
+                                  pv(m, st, 6), k->groups[6], beta, m->dt, s);
+  ctx->mark_end(s);
+  if (learned) {
+    launch_c2p(m, st, 6, s, true);
+    launch_c2p_queued(m, st, "con2prim_learned_first", s);
+  }
   ctx->mark_begin("c2p_fixup", s);
   launch_pack_c2p_fixup(k->p.geom.kind, k->dp, k->fx, pv(m, st, 4), k->groups[4], s);
   ctx->mark_end(s);
