@@ -127,12 +127,18 @@ __device__ __forceinline__ double xf(const BlockGeom &b, int d, int idx) {
 // its exact remainder.  They give the IEEE results wherever no intermediate leaves the normal
 // range (|b| and |a / b| within 2^+-960, |a| above 2^-900 or zero; compared with the
 // compiler's a / b and sqrt on 2^24 operands with exponents within +-380 and +-900), and
-// div_fixup / the class test give the special cases (zeros, infinities, NaN).  The
-// compiler's sequences also scale operands near the ends of the range, which nothing in
-// the fluid path reaches: 70 and 90 issue cycles of a SIMD per wave against 56 and 66 here, and a
-// further quotient by the same denominator costs 18 (its reciprocal is one common
-// subexpression).  The sweeps of the exact arithmetic spend a fifth of their instructions in
-// divisions and the root find half of its time.
+// div_fixup / the class test give the special cases: zeros, infinities, NaN, and a quotient
+// that overflows (its NaN estimate from finite operands becomes the infinity).  Beyond that
+//   a subnormal denominator gives an infinity: where one can occur (a density, a pressure or a
+//   floor that no minimum bounds) the code divides with /;
+//   a numerator below 2^-969 leaves the quotient up to two units in the last place off;
+//   a radicand below 2^-969 gives a root within 2^-47: the code takes sqrt where one can occur.
+// The compiler's sequences scale the operands first: 70 and 90 issue cycles of a SIMD per wave
+// against 56 and 66 here, and a further quotient by the same denominator costs 18 (its reciprocal
+// is one common subexpression).  The sweeps of the exact arithmetic spend a fifth of their
+// instructions in divisions and the root find half of its time; the dozen divisions by / per
+// zone or face are below what a stage's time resolves (128^3 835 / 838 us, 64^3 tasks 225 / 226,
+// 2^22 inversions 386 / 386).
 __device__ __forceinline__ double refined_rcp(double b) {
   double y = __builtin_amdgcn_rcp(b);
   y = fma(fma(-b, y, 1.0), y, y);
@@ -677,7 +683,7 @@ __device__ __forceinline__ Floors floors_at(const DevBounds &b, double x1, doubl
 }
 __device__ __forceinline__ double sie_floor_of(const DevBounds &b, const Floors &f, double rho) {
   return b.floor_type == PHX_FLOOR_EXPX1_RHO_U
-             ? smax(ddiv(f.sie, smax(rho, f.den)), b.sie_min_eos)
+             ? smax(f.sie / smax(rho, f.den), b.sie_min_eos)
              : f.sie;
 }
 
@@ -721,14 +727,15 @@ __device__ __forceinline__ void prim_to_flux(const DevParams &p, const int dir, 
       if (M::nz_cov(ii + 1, jj + 1)) vsq0 += g.gcov(ii + 1, jj + 1) * vpcon[ii] * vpcon[jj];
   double W = fsqrt(1. + vsq0);
   if (W > gam_max) {
-    const double rescale = fsqrt(fdiv(gam_max * gam_max - 1., W * W - 1.));
+    const double gg = gam_max * gam_max - 1., ww = W * W - 1.;  // their ratio may be tiny
+    const double rescale = kFluxFast ? fsqrt(fdiv(gg, ww)) : sqrt(gg / ww);
 #pragma unroll
     for (int ii = 0; ii < 3; ++ii) vpcon[ii] *= rescale;
   }
   double vcon[3] = {fdiv(vpcon[0], W), fdiv(vpcon[1], W), fdiv(vpcon[2], W)};
   const double vel = vcon[dir];
   double Bcon[3] = {0.0, 0.0, 0.0};
-  const double sie = ddiv(q[4], rho);
+  const double sie = q[4] / rho;  // rho may be zero or subnormal where no floor acts
   const double u = (sie > sie_floor ? (sie > sie_max ? rho * sie_max : q[4]) : rho * sie_floor);
   const double P = smax(q[L::prs], 0.0);
   const double gamma1 = q[L::gm1];
@@ -955,9 +962,9 @@ template <class M>
 __device__ __forceinline__ void signal_speeds(double rho, double u, double pr, double bsq,
                                               const double v[3], double vsq, double gam1,
                                               const M &g, double sig[3]) {
-  const double rho_rel = rho + u + pr;
-  const double vasq = ddiv(bsq, rho_rel + bsq);
-  double cssq = ddiv(gam1 * pr, rho_rel);
+  const double rho_rel = rho + u + pr;  // subnormal in an evacuated zone
+  const double vasq = bsq / (rho_rel + bsq);
+  double cssq = gam1 * pr / rho_rel;
   cssq += vasq - cssq * vasq;
   const double vcoff = ddiv(g.alpha(), 1.0 - vsq * cssq);
 #pragma unroll
@@ -1195,7 +1202,7 @@ __device__ __forceinline__ bool c2p_setup(const DevParams &p, const M &g, const 
   if constexpr (MHD) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) prim[5 + i] = cons[5 + i] * igdet;
-    const double sD = ddiv(1.0, dsqrt(smax(D, rhoflr)));
+    const double sD = ddiv(1.0, sqrt(smax(D, rhoflr)));
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       z.bu[i] = prim[5 + i] * sD;
@@ -1243,7 +1250,7 @@ __device__ __forceinline__ double c2p_unwrap(const DevParams &p, const M &g, C2P
   temp = eos_t_rho_sie(p, prim[4]);
   prim[4] *= prim[0];
   prim[L::prs] = eos_p_rho_t(p, prim[0], temp);
-  prim[L::gm1] = ddiv(eos_bmod_rho_t(p, prim[0], temp), prim[L::prs]);
+  prim[L::gm1] = eos_bmod_rho_t(p, prim[0], temp) / prim[L::prs];
   double vel[3], bu[3] = {z.bu[0], z.bu[1], z.bu[2]};
 #pragma unroll
   for (int i = 0; i < 3; ++i) {

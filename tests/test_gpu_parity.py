@@ -264,6 +264,78 @@ def test_division_range_bits(phx, scale, mhd):
                 assert np.array_equal(gf[d, m][sl], rf[d, m][sl], equal_nan=True), (recon, d, m)
 
 
+EVACUATED = {  # floors and ceilings
+    "none": {},
+    "floors": dict(floors=dict(rho0=1e-7, sie0=1e-5), ceilings=(50.0, 100.0)),
+    "ceilings": dict(ceilings=(50.0, 100.0)),
+    "rho_u": dict(floors=dict(floor_type=A.FLOOR_EXPX1_RHO_U, rho0=1e-7, sie0=1e-9,
+                              rho_exp=-2.0, sie_exp=-3.0), ceilings=(50.0, 100.0)),
+    "subnormal": dict(floors=dict(floor_type=A.FLOOR_EXPX1_RHO_U, rho0=1e-310, sie0=1e-5,
+                                  rho_exp=-2.0, sie_exp=-3.0), ceilings=(1e30, 1e300)),
+}
+
+
+@pytest.mark.parametrize("mhd", [False, True])
+@pytest.mark.parametrize("bounds", EVACUATED)
+def test_evacuated_zones_bits(phx, bounds, mhd):
+    """Zones with no mass, or a subnormal density or pressure, equal the oracle's bits: the
+    inversion with tau / D on both sides of overflow, and the fluxes of such primitives."""
+    say(f"[gpu] evacuated zones bounds={bounds} mhd={mhd}")
+    states = np.array([(d, t, s, b)
+                       for d in (0.0, -0.0, 5e-324, 1e-310, 2.3e-308, 1e-307, 1e-300, 1e-150, 1.0)
+                       for t in (0.0, 1e-300, 1e-150, 1.0, 39.0, 41.0, 50.0, 1e6, 1e150, 1e300, -1.0)
+                       for s in (0.0, 1e-300, 1e-10, 1.0)
+                       for b in ((0.0, 1e-160, 1e-3, 1.0) if mhd else (0.0,))]).T
+    n = states.shape[1]
+    cons = np.zeros((8 if mhd else 5, n))
+    cons[0], cons[4], cons[1], cons[3] = states[0], states[1], states[2], -0.5 * states[2]
+    if mhd:
+        cons[5], cons[6] = states[3], 0.25 * states[3]
+    p = fluid_params(gamma=4.0 / 3.0, mhd=mhd, **EVACUATED[bounds])
+    op = oparams(p)
+    for mu0 in (0.0, 0.5):
+        with np.errstate(all="ignore"):
+            ref = O.c2p_batch(op, np.zeros((2, n)), cons, np.full(n, mu0))
+        d_cons, d_prim = DeviceArray.from_host(cons), DeviceArray(ref["prim"].shape)
+        d_prim.zero()
+        d_mu, d_fail = DeviceArray.from_host(np.full(n, mu0)), DeviceArray((n,))
+        d_it = DeviceArray((n,), np.int32)
+        phx.con2prim_batch(p, n, None, d_cons, d_prim, d_mu, d_fail, d_it)
+        synchronize()
+        assert np.array_equal(d_fail.get(), ref["fail"])
+        assert np.array_equal(d_it.get(), ref["iters"])
+        assert np.array_equal(d_mu.get(), ref["mu"], equal_nan=True)
+        assert np.array_equal(d_prim.get(), ref["prim"], equal_nan=True)
+        good = ref["fail"] == 1.0  # (a zone that fails keeps what its re-derivation left)
+        assert np.array_equal(d_cons.get()[:, good], ref["cons"][:, good], equal_nan=True)
+    if "floor_type" in EVACUATED[bounds].get("floors", {}):
+        return  # exp(x1) of a block's faces is the device library's (at the states' x1 = 0 it is 1)
+    rng = np.random.default_rng(11)
+    b = geom_block(3, (11, 9, 8), A.GEOM_MINKOWSKI)
+    sh = O.block_shape(oblock(b))
+    prim = random_block(rng, b, mhd, 4.0 / 3.0, A.GEOM_MINKOWSKI)
+    for v in (0, 4, prim.shape[0] - 2):  # rho, u, P
+        prim[v] = rng.choice([0.0, 5e-324, 1e-310, 2.3e-308, 1e-300, 1e-20, 1.0], sh)
+    fast = rng.random(sh) < 0.1
+    prim[1:4] = np.where(fast, 1e150 * np.sign(prim[1:4]), prim[1:4])
+    for recon in (A.RECON_CONSTANT, A.RECON_LINEAR):
+        for solver in (A.RIEMANN_HLL, A.RIEMANN_LLF):
+            q = fluid_params(gamma=4.0 / 3.0, mhd=mhd, recon=recon, riemann=solver,
+                             **EVACUATED[bounds])
+            rf, rs = O.calculate_fluxes(oparams(q), oblock(b), prim)
+            st = BlockState(q, b)
+            st.prim.upload(prim)
+            phx.calculate_fluxes(q, b, st.fields())
+            synchronize()
+            gf, gs = st.flux.get(), st.face_sig.get()
+            for d in range(3):
+                sl = consumed_face_slices(b, d)
+                assert np.array_equal(gs[d][sl], rs[d][sl], equal_nan=True), (recon, solver, d)
+                for m in range(rf.shape[1]):
+                    assert np.array_equal(gf[d, m][sl], rf[d, m][sl], equal_nan=True), \
+                        (recon, solver, d, m)
+
+
 def test_batch_edge_sizes(phx):
     # an empty batch is a no-op (no pointer is read), a negative one is refused, and ragged
     # sizes (not multiples of a wave or a 256-lane group) match the oracle bit for bit and
