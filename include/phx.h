@@ -24,10 +24,14 @@
  *    con2prim_robust.hpp:41-44).
  *  - No entry point allocates device memory after phx_create; scratch lives in the
  *    context.  A context is bound to one device and is not thread-safe.
- *  - The context's scratch (the CFL partial minima written by phx_fluid_stage and
- *    phx_estimate_dt when dt_out is set) is one buffer per context: calls that use it
- *    must be ordered, i.e. issued on one stream, or on streams the caller orders with
- *    events.  Two such calls in flight at once on different streams race on it.
+ *  - The context's scratch (CFL partial minima, which phx_fluid_stage and phx_estimate_dt
+ *    may write when dt_out is set) is one buffer per context: calls with dt_out set must be
+ *    ordered, i.e. issued on one stream, or on streams the caller orders with events.  Two
+ *    such calls in flight at once on different streams race on it, or on a dt_out that they
+ *    share: a stage may set dt_out early and lower it cell by cell, so it holds the time
+ *    step only once the call's last launch has ended.
+ *  - dt_out is one double in device memory or in host memory that the device can write
+ *    (hipHostMalloc, managed).
  */
 #ifndef PHX_H_
 #define PHX_H_
@@ -205,7 +209,7 @@ int phx_con2prim(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
                  const phx_block_fields *f, const int lo[3], const int hi[3], int32_t *iters,
                  phx_stream stream);
 
-/* fluid::EstimateTimestepBlock (fluid.cpp:899-944): dt_out[0] (device) = cfl * min over
+/* fluid::EstimateTimestepBlock (fluid.cpp:899-944): dt_out[0] = cfl * min over
  * interior cells.  use_face_speeds = 0 selects the reference's first-call form
  * (cell speeds only, :930-939). */
 int phx_estimate_dt(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
@@ -229,7 +233,7 @@ int phx_estimate_dt(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
  * CalculateFluxes; phx_flux_ct on f afterwards gives the rewritten ones.
  * f->cons is U_s (averaged in place); writes a->u_out (U_{s+1}, after any con2prim
  * re-synchronisation), a->prim_out (may alias f->prim), f->temp, f->c2p_mu, f->cell_sig,
- * f->fail and, when non-NULL, a->iters and a->dt_out (device; cfl * min over the block,
+ * f->fail and, when non-NULL, a->iters and a->dt_out (cfl * min over the block,
  * with face speeds as fluid.cpp:913-928).  Bit-identical to the separate task entry
  * points called in the same order. */
 typedef struct {
@@ -239,7 +243,7 @@ typedef struct {
   double *prim_out;      /* [nprim][cells]; may alias f->prim                   */
   int32_t *iters;        /* [cells] con2prim iterations, nullable               */
   double cfl;
-  double *dt_out;        /* [1] device, nullable                                */
+  double *dt_out;        /* [1] nullable                                       */
   /* per-component overrides (as phx_block_fields::vars), nullable: base_vars->cons for
    * u_base; out_vars->cons for u_out and out_vars->prim for prim_out */
   const phx_block_vars *base_vars, *out_vars;

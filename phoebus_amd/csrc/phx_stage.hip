@@ -214,8 +214,8 @@ __device__ __forceinline__ void lower_to(double *q, double v) {
 }
 
 // The CFL time goes to dt, which the corner EMFs' launch set to its largest value, or its partial
-// minima to partial (no such launch, or cfl <= 0: cfl > 0 scales before the minimum as it does
-// after it, since rounding keeps the order).  Without the finishing launch a stage of 16^3 cells
+// minima to partial (no such launch, dt not in plain device memory, or cfl <= 0: cfl > 0 scales
+// before the minimum as it does after it, since rounding keeps the order).  Without the finishing launch a stage of 16^3 cells
 // takes 33.3 instead of 34.6 us, 256x128 on Kerr-Schild 39.3 / 40.1, 64x64x32 on FMKS 157.9 /
 // 159.1, 128^3 the same; with exchanges instead of the minimum instruction only 16^3 gained.
 template <bool MHD, int GEOM, int NDIM>
@@ -391,6 +391,21 @@ int static_scratch(double **out) {
 const char *noalloc_last_error() { return g_noalloc_err; }
 }  // namespace phx
 
+// Whether q is in plain (coarse-grained) memory of the current device, where the 64-bit minimum
+// of lower_to is defined: PCIe has no such atomic operation, so in host memory, in managed and
+// in fine-grained memory a call may lose it.  The runtime's look-up takes 0.06 us and is legal
+// during a capture.
+static bool in_device_memory(const double *q) {
+  hipPointerAttribute_t at;
+  int dev = -1;
+  if (hipPointerGetAttributes(&at, q) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return at.type == hipMemoryTypeDevice && !at.isManaged && at.allocationFlags == 0 &&
+         hipGetDevice(&dev) == hipSuccess && at.device == dev;
+}
+
 // the stage's launches; partial = the CFL partial minima buffer (at least kDtPartials)
 static int fluid_stage_launches(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
                                 const phx_block_fields *f, const phx_stage_args *a,
@@ -434,7 +449,7 @@ static int fluid_stage_launches(phx_ctx *ctx, const phx_fluid_params *p, const p
     ctx->mark_end(s);
   }
   const bool ct = p->mhd && b->ndim > 1;
-  const bool dt_direct = a->dt_out && ct && a->cfl > 0.0;
+  const bool dt_direct = a->dt_out && ct && a->cfl > 0.0 && in_device_memory(a->dt_out);
   // FluxCT: the EMFs here, the B-flux rewrite in the update
   double *dt = dt_direct ? a->dt_out : nullptr;
   if (ct && curved) {

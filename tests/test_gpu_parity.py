@@ -5,6 +5,7 @@ library and the oracle round +,-,*,/,sqrt identically with contraction off); cur
 metrics within 1e-12 relative (sin/cos differ by an ulp between the device math library
 and glibc).  Flux comparisons cover the faces the stage consumes.
 """
+import ctypes as C
 import sys
 
 import numpy as np
@@ -794,6 +795,68 @@ def test_stage_dt_is_that_of_its_speeds(phx, nx, mhd, cfl):
         assert out.get()[0] == want.get()[0]
         got.append(out.get()[0])
     assert got[0] == got[2] and (cfl == 0.0 or got[1] != got[0])  # one rise, one fall
+
+
+def launch_names(phx, call):
+    """The names of the launches that call() marks in the context."""
+    L, n, ms, name = phx.L, C.c_int(), C.c_float(), C.create_string_buffer(64)
+    L.phx_rt_profile_start(phx.h)
+    L.phx_rt_profile_reset(phx.h)
+    call()
+    synchronize()
+    L.phx_rt_profile_count(phx.h, C.byref(n))
+    out = []
+    for i in range(n.value):
+        assert L.phx_rt_profile_get(phx.h, i, name, 64, C.byref(ms)) == 0
+        out.append(name.value.decode())
+    L.phx_rt_profile_stop(phx.h)
+    return out
+
+
+class HipScalar:
+    """One double from another allocator of the HIP runtime (pinned host memory, fine-grained
+    device memory)."""
+
+    def __init__(self, kind):
+        self.hip, p = A.lib(), C.c_void_p()  # dlsym finds the runtime behind the library
+        rc = {"pinned": lambda: self.hip.hipHostMalloc(C.byref(p), C.c_size_t(8), C.c_uint(0)),
+              "noncoherent": lambda: self.hip.hipHostMalloc(C.byref(p), C.c_size_t(8),
+                                                            C.c_uint(0x80000000)),
+              "finegrained": lambda: self.hip.hipExtMallocWithFlags(
+                  C.byref(p), C.c_size_t(8), C.c_uint(1))}[kind]()
+        assert rc == 0
+        self.host, self.ptr, self.nbytes = kind != "finegrained", p.value, 8
+
+    def get(self):
+        v = C.c_double()
+        assert self.hip.phx_rt_memcpy_dtoh(C.addressof(v), self.ptr, 8) == 0
+        return v.value
+
+    def free(self):
+        f = self.hip.hipHostFree if self.host else self.hip.hipFree
+        assert f(C.c_void_p(self.ptr)) == 0
+
+
+@pytest.mark.parametrize("kind", ["pinned", "noncoherent", "finegrained"])
+@pytest.mark.parametrize("geom", [A.GEOM_MINKOWSKI, A.GEOM_SPHERICAL_KS])
+def test_stage_dt_outside_plain_device_memory(phx, kind, geom):
+    """dt_out where 64-bit atomic minima are not defined: the finishing launch writes it, with
+    the value that plain device memory gets."""
+    say(f"[gpu] stage dt in {kind} memory, geom {geom}")
+    b = geom_block(3, (18, 10, 9), geom)
+    p = geom_params(geom, gamma=4.0 / 3.0, mhd=True, recon=A.RECON_WENO5Z,
+                    riemann=A.RIEMANN_HLL)
+    st = BlockState(p, b)
+    st.prim.upload(random_block(np.random.default_rng(3), b, True, 4.0 / 3.0, geom))
+    phx.prim_to_con(p, b, st.fields())
+    u_out, prim_out = DeviceArray(st.cons.shape), DeviceArray(st.prim.shape)
+    there, plain = HipScalar(kind), DeviceArray((1,))
+    names = [launch_names(phx, lambda: phx.fluid_stage(
+        p, b, st.fields(with_src=True), 1.0, 1e-4, st.cons, u_out, prim_out, cfl=0.4, dt_out=out))
+        for out in (plain, there)]
+    assert there.get() == plain.get()[0] > 0.0
+    assert "dt_finish" not in names[0] and "dt_finish" in names[1]
+    there.free()
 
 
 @pytest.mark.parametrize("geom", [A.GEOM_SPHERICAL_KS, A.GEOM_FMKS])
