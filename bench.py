@@ -83,8 +83,12 @@ def kernel_bytes(nx):
     flux_dir = faces * (10 + 8 + 1) * 8  # 10 primitives in, 8 fluxes + 1 speed out
     return {
         "flux_x": flux_dir, "flux_y": flux_dir, "flux_z": flux_dir,
+        "flux_xyz": 3 * flux_dir,  # the sweeps of a block in one launch
         # FluxCT's EMF pass: 6 transverse B fluxes in, 3 corner EMFs out
         "flux_ct": (nx + 1) ** 3 * (6 + 3) * 8,
+        # curved metrics: 9 primitives in, 4 sources out, alone and with the EMF pass
+        "sources": cells * (9 + 4) * 8,
+        "sources_ct": cells * (9 + 4) * 8 + (nx + 1) ** 3 * (6 + 3) * 8,
         # 18 face fluxes (the B fluxes come from the EMFs), 3 EMFs, U_s, U^n, mu, 3 face
         # speeds in; U_s, U_{s+1}, 10 prims, T, mu, fail, 3 cell speeds, int32 iteration
         # count out
@@ -947,7 +951,9 @@ def c2_stage(phx, args, recon_name, prim_h, step, full=True, arith=None):
     value = nx ** 3 / (ms_per_step * 1e-3)
     leg = {"flux_arith": arith, "ms_per_step": ms_per_step, "zone_updates_per_s": value,
            "stage_hbm_frac": value * B_ALG_STAGE / 1e9 / HBM_PEAK_GBS,
-           "dt": dt, "flux_tiles_yz": tiles, "launch_ms": launch_ms,
+           "dt": dt, "launch_ms": launch_ms,
+           # (the sweeps of a block in one launch have no y and z shapes of their own)
+           "flux_tiles_yz": None if "flux_xyz" in launch_ms else tiles,
            "con2prim_mean_iters_warm": float(np.mean(warm_iters)),
            "fail_count": int(np.sum(st.fail.get()[I] == 0.0))}
     if not full:

@@ -51,3 +51,23 @@ def test_stage_profile_digest_covers_every_sweep_unit():
     for f in listed:
         assert os.path.exists(os.path.join(ROOT, f)), f
     assert len(bench.sources_digest()) == 64
+
+
+def test_every_stage_launch_has_its_bytes():
+    """The roofline leg looks the stage's longest launch up by name: every name that the fused
+    stage can mark has an entry."""
+    import importlib.util
+    import re
+
+    spec = importlib.util.spec_from_file_location("bench_mod", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    src = open(os.path.join(ROOT, "phoebus_amd", "csrc", "phx_stage.hip")).read()
+    names = set(re.findall(r'mark_begin\("(\w+)"', src))
+    table = re.search(r"kFluxName\[\d+\] = \{([^}]*)\}", src).group(1)
+    names |= set(re.findall(r'"(\w+)"', table))
+    assert {"flux_x", "flux_y", "flux_z", "flux_xyz", "update_con2prim", "dt_finish"} <= names
+    kb = bench.kernel_bytes(16)
+    for name in sorted(names):
+        assert kb.get(name, 0) > 0, name
+    assert kb["flux_xyz"] == kb["flux_x"] + kb["flux_y"] + kb["flux_z"]
