@@ -293,12 +293,16 @@ int phx_prim_to_con_batch(phx_ctx *ctx, const phx_fluid_params *p, int64_t n,
  * then use it.  A shape (ti, ts) with ts > 0 is a tile of ti cells along i by ts along
  * the sweep; with ts < 0, one 64-lane wave of ti columns (a power of two) by 64 / ti rows
  * marching along the sweep in -ts segments of the faces.  Results do not depend on the
- * shape.  reps = timed launches per candidate.  phx_tile_shape reports the shape in use
- * for dir 1 (y) or 2 (z); phx_set_tile_shape fixes one (ts = 0: the default, marching waves
- * of 8 x 8 or tiles of 8 x 32, whichever takes fewer wave-steps on the block; tiles for
- * the constant and linear reconstructions).  While a block's shapes are the defaults, the
- * sweeps of all directions go in one launch where that is faster (small blocks, and any
- * block with the constant and linear reconstructions); phx_autotune times that too. */
+ * shape.  reps = timed launches per candidate.  phx_tile_shape reports the shape of the
+ * launch of its own that dir 1 (y) or 2 (z) takes; phx_set_tile_shape fixes it (ts = 0: the
+ * default, marching waves of 8 x 8 or tiles of 8 x 32, whichever takes fewer wave-steps on
+ * the block; tiles for the constant and linear reconstructions).  While a block's shapes are
+ * the defaults, the sweeps of all directions go in one launch where that is faster (small
+ * blocks, and any block with the constant and linear reconstructions): y and z then have no
+ * launch of their own and run tiles of up to 8 x 32 in it, whatever phx_tile_shape reports,
+ * and the stage marks one launch flux_xyz (phx_rt_profile_get) in place of flux_x, flux_y and
+ * flux_z.  Fixing a shape, the reported default too, gives up the one launch.  phx_autotune
+ * times both and, where the one launch wins, leaves the defaults. */
 int phx_autotune(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
                  const phx_block_fields *f, int reps, phx_stream stream);
 int phx_tile_shape(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b, int dir,

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import _physics as PH
+from _launches import launch_names
 from phoebus_amd import _abi as A
 from phoebus_amd.api import BlockState, Pack, Phx, block, fixup_params, fluid_params, mgr
 from phoebus_amd.device import DeviceArray, synchronize
@@ -151,6 +152,46 @@ def test_pack_matches_single_block_stages(phx, geom, sizes):
     assert dt2 == min(dts2)
     fails = sum(int(np.sum(s[4][4:-4, 4:-4, 4:-4] == 0.0)) for s in after2)
     say(f"    con2prim failures after stage 2: {fails}")
+    pk.close()
+
+
+@pytest.mark.parametrize("geom", [A.GEOM_MINKOWSKI, A.GEOM_FMKS])
+def test_marching_pack_matches_marching_and_merged_single_blocks(phx, geom):
+    """A pack's marching y/z sweeps against a single block's: marching by fixed shapes, and in
+    the one launch of its defaults.  phx_tile_shape gives the shape of a direction's own
+    launch, which a block takes once it is fixed."""
+    say(f"[gpu] marching pack vs marching and merged single-block sweeps, geom {geom}")
+    p = _params(geom)
+    blocks = _blocks(geom, MARCH_SIZES)
+    S = Setup(phx, p, blocks, np.random.default_rng(13 + geom), geom)
+    pk = Pack(phx, p, [(b, st, c1, it) for b, st, c1, it in
+                       zip(blocks, S.states, S.cons1, S.iters)])
+    assert all(pk.tile_shape(d)[1] < 0 for d in (1, 2))
+    S.reset()
+    pk.stage(1, dt=1e-3)
+    synchronize()
+    want = S.snapshot()
+    curved = geom != A.GEOM_MINKOWSKI
+    for fixed in (False, True):
+        if fixed:
+            for b in blocks:
+                for d in (1, 2):
+                    ti, ts = phx.tile_shape(p, b, d)
+                    phx.set_tile_shape(p, b, d, ti, ts if ts < 0 else -2)
+
+        def stages():
+            for b, st, c1, it in zip(blocks, S.states, S.cons1, S.iters):
+                phx.fluid_stage(p, b, st.fields(with_src=curved), 1.0, 1e-3, st.cons, c1, st.prim,
+                                iters=it)
+
+        S.reset()
+        names = launch_names(phx, stages)
+        assert names.count("flux_xyz") == (0 if fixed else len(blocks))
+        assert names.count("flux_y") == names.count("flux_z") == (len(blocks) if fixed else 0)
+        _equal(S.snapshot(), want, "fixed" if fixed else "default")
+    for b in blocks:
+        for d in (1, 2):
+            phx.set_tile_shape(p, b, d, 0, 0)
     pk.close()
 
 

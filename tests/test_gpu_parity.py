@@ -13,6 +13,7 @@ import pytest
 
 import _oracle as O
 import _physics as PH
+from _launches import launch_names
 from phoebus_amd import _abi as A
 from phoebus_amd.api import BlockState, Phx, block, fluid_params, mgr
 from phoebus_amd.device import DeviceArray, synchronize
@@ -795,22 +796,6 @@ def test_stage_dt_is_that_of_its_speeds(phx, nx, mhd, cfl):
         assert out.get()[0] == want.get()[0]
         got.append(out.get()[0])
     assert got[0] == got[2] and (cfl == 0.0 or got[1] != got[0])  # one rise, one fall
-
-
-def launch_names(phx, call):
-    """The names of the launches that call() marks in the context."""
-    L, n, ms, name = phx.L, C.c_int(), C.c_float(), C.create_string_buffer(64)
-    L.phx_rt_profile_start(phx.h)
-    L.phx_rt_profile_reset(phx.h)
-    call()
-    synchronize()
-    L.phx_rt_profile_count(phx.h, C.byref(n))
-    out = []
-    for i in range(n.value):
-        assert L.phx_rt_profile_get(phx.h, i, name, 64, C.byref(ms)) == 0
-        out.append(name.value.decode())
-    L.phx_rt_profile_stop(phx.h)
-    return out
 
 
 class HipScalar:
