@@ -30,18 +30,30 @@ TileShape pack_shape(const phx_pack *k, int d, TileShape want) {
   return best;
 }
 
-// the shape a pack starts with: its blocks share the launch, so the march needs fewer segments
+// the marching waves of direction d over the pack
+static long pack_waves(const phx_pack *k, int d, TileShape t) {
+  long waves = 0;
+  for (const auto &g : k->geoms) waves += pack_groups_flux(d, k->p.recon, g, t);
+  return waves;
+}
+
+// The shape a pack starts with: its blocks share the launch, so the march needs fewer segments
 // than each block's own default would take: the fewest that make two rounds of four waves per
 // SIMD over the pack, up to 8 (40 FMKS torus blocks, y / z sweep: 8 x -1, 6120 waves, 300 /
-// 301 us; 8 x -2 258 / 253); tiles where the stencil is short, as for single blocks
+// 301 us; 8 x -2 258 / 253).  With the short stencils a wave-step hardly pays for the ring, so
+// two segments where they make 6,000 waves, else tiles: two RK2 steps in PLM (us, march /
+// tiles) of 8 64^3 blocks (8,712 waves) 3499 / 3723 on Minkowski and 4154 / 4363 on FMKS,
+// 27 32^3 (7,803) 1904 / 2120; 64 16^3 (5,184) 1086 / 1095, in constant reconstruction on FMKS
+// 1337 / 1306; one 128^3 (4,225) 3472 / 3245, 16 16^3 (1,296) 370 / 353.
 static TileShape pack_default_shape(const phx_pack *k, int d) {
-  if (k->p.recon < PHX_RECON_WENO5Z) return pack_shape(k, d, TileShape{8, 32});
+  if (k->p.recon < PHX_RECON_WENO5Z) {
+    const TileShape m = pack_shape(k, d, TileShape{8, -2});
+    return pack_waves(k, d, m) >= 6000 ? m : pack_shape(k, d, TileShape{8, 32});
+  }
   TileShape t;
   for (int nseg = 1; nseg <= 8; ++nseg) {
     t = pack_shape(k, d, TileShape{8, -nseg});
-    long waves = 0;
-    for (const auto &g : k->geoms) waves += pack_groups_flux(d, k->p.recon, g, t);
-    if (waves >= 8192) break;
+    if (pack_waves(k, d, t) >= 8192) break;
   }
   return t;
 }

@@ -195,6 +195,33 @@ def test_marching_pack_matches_marching_and_merged_single_blocks(phx, geom):
     pk.close()
 
 
+@pytest.mark.parametrize("geom", [A.GEOM_MINKOWSKI, A.GEOM_FMKS])
+@pytest.mark.parametrize("recon", [A.RECON_CONSTANT, A.RECON_LINEAR])
+def test_short_stencil_pack_defaults(phx, recon, geom):
+    """With the constant and linear reconstructions a pack's sweep marches by default where two
+    segments make 6,000 waves (y here) and runs tiles elsewhere (z); both match the single-block
+    stage."""
+    say(f"[gpu] default shapes of a pack, recon {recon} geom {geom}")
+    p = _params(geom)
+    p.recon = recon
+    blocks = _blocks(geom, [(64, 4, 64)] * 6)
+    S = Setup(phx, p, blocks, np.random.default_rng(7 + geom), geom)
+    pk = Pack(phx, p, [(b, st, c1, it) for b, st, c1, it in
+                       zip(blocks, S.states, S.cons1, S.iters)])
+    assert pk.tile_shape(1) == (8, -2) and pk.tile_shape(2)[1] > 0
+    S.reset()
+    pk.stage(1, dt=1e-3)
+    synchronize()
+    got = S.snapshot()
+    S.reset()
+    for b, st, c1, it in zip(blocks, S.states, S.cons1, S.iters):
+        phx.fluid_stage(p, b, st.fields(with_src=geom != A.GEOM_MINKOWSKI), 1.0, 1e-3, st.cons, c1,
+                        st.prim, iters=it)
+    synchronize()
+    _equal(S.snapshot(), got, "stage 1")
+    pk.close()
+
+
 def test_pack_graph_replays_match_eager(phx):
     say("[gpu] pack graph (two stages, device dt) replayed 3x vs eager")
     geom = A.GEOM_MINKOWSKI
