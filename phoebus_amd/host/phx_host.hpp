@@ -91,8 +91,9 @@ namespace update {
 // phoebus_driver.cpp:560-576: containers by index
 TaskStatus FluxDivergenceUpdate(MeshBlockData *rc, int stage_container, int base_container,
                                 double beta, double dt, int out_container);
-// fluid::FluxCT (its corner EMFs; the shared flux field keeps the Riemann solver's magnetic
-// fluxes), FluxDivergenceUpdate and fluid::ConservedToPrimitive of the out container
+// What the driver runs in place of fluid::FluxCT (its corner EMFs; the shared flux field keeps the
+// Riemann solver's magnetic fluxes), FluxDivergenceUpdate and fluid::ConservedToPrimitive of the
+// out container: the same bits
 TaskStatus UpdateFillDerived(MeshBlockData *rc, int stage_container, int base_container,
                              double beta, double dt, int out_container);
 }  // namespace update
