@@ -218,11 +218,13 @@ int phx_estimate_dt(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
 
 /* ---- one RK stage --------------------------------------------------------------------
  * The fluid tasks of one stage of PhoebusDriver::RungeKuttaStage (phoebus_driver.cpp:
- * 330-722) for one block, fused into five launches: CalculateFluxes (:344), FluxCT's
- * corner EMFs (:345), CalculateFluidSourceTerms (:322, curved metrics only), then
- * FluxCT's rewrite of the B fluxes, FluxDivergence + SumData + AverageIndependentData +
- * UpdateIndependentData (:560-576) fused with the robust ConservedToPrimitive
- * (FillDerived, :588) and the CFL reduction (:720-722) in one kernel.
+ * 330-722) for one block, fused into five launches, three where the sweeps go in one (see
+ * phx_tile_shape): CalculateFluxes (:344), FluxCT's corner EMFs (:345) with
+ * CalculateFluidSourceTerms (:322, curved metrics only), then FluxCT's rewrite of the B
+ * fluxes, FluxDivergence + SumData + AverageIndependentData + UpdateIndependentData
+ * (:560-576) fused with the robust ConservedToPrimitive (FillDerived, :588) and the CFL
+ * reduction (:720-722) in one kernel.  Without CT, for cfl <= 0 and for a dt_out outside plain
+ * device memory one more launch finishes the reduction.
  * con2prim runs on the interior cells: the ghost zones are refilled by the boundary
  * exchange and re-inverted there (:646-668), which this call does not cover.
  *
@@ -257,7 +259,7 @@ int phx_fluid_stage(phx_ctx *ctx, const phx_fluid_params *p, const phx_block *b,
  * create a context on the calling path (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  The same launches and results as phx_fluid_stage,
  * bit for bit, with the built-in default sweep shapes (no autotuned shape: there is no
- * context).  The CFL partial minima go to a file-scope device array of 65536 doubles
+ * context).  CFL partial minima, where used, go to a file-scope device array of 65536 doubles
  * (512 KiB) that each device holds from its first use until the process ends; its address
  * is looked up by phx_create, or by the first call on a device with that device current.
  * Call with the stream's device current (stream NULL = that device's null stream).

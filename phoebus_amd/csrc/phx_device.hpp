@@ -164,7 +164,9 @@ __device__ __forceinline__ double dsqrt(double x) {
   g = fma(fma(-g, g, x), h, g);
   return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +-0 and +inf are their own roots
 }
-// for x in [0, 1] (or NaN): only zero needs care, and a bounded estimate makes its root 0
+// for x in [0, 1] (or NaN): only zero needs care, and a bounded estimate makes its root 0.  (The
+// root find's radicand is negative only where r^2 is infinite; the -inf that it gets then
+// makes the residual the NaN that sqrt's would.)
 __device__ __forceinline__ double dsqrt_unit(double x) {
   const double y = fmin(__builtin_amdgcn_rsq(x), 0x1p512);
   double g = x * y, h = 0.5 * y;
@@ -222,6 +224,15 @@ __device__ __forceinline__ double fdiv(double a, double b) {
     return a * frcp(b);
   else
     return ddiv(a, b);
+}
+// a / b where b may be subnormal: as /, or in the fast arithmetic scaled first, which is exact and
+// serves magnitudes below 2^962 (with / the fast sweeps ran 1-2 % slower: the longer sequences
+// move what the compiler keeps in SGPRs)
+__device__ __forceinline__ double div_any(double a, double b) {
+  if constexpr (kFluxFast)
+    return ddiv(a * 0x1p60, b * 0x1p60);
+  else
+    return a / b;
 }
 // fdiv where the denominator is positive and finite (the WENO weights: an infinite
 // smoothness indicator makes the edge NaN with either)
@@ -683,7 +694,7 @@ __device__ __forceinline__ Floors floors_at(const DevBounds &b, double x1, doubl
 }
 __device__ __forceinline__ double sie_floor_of(const DevBounds &b, const Floors &f, double rho) {
   return b.floor_type == PHX_FLOOR_EXPX1_RHO_U
-             ? smax(f.sie / smax(rho, f.den), b.sie_min_eos)
+             ? smax(div_any(f.sie, smax(rho, f.den)), b.sie_min_eos)
              : f.sie;
 }
 
@@ -735,7 +746,7 @@ __device__ __forceinline__ void prim_to_flux(const DevParams &p, const int dir, 
   double vcon[3] = {fdiv(vpcon[0], W), fdiv(vpcon[1], W), fdiv(vpcon[2], W)};
   const double vel = vcon[dir];
   double Bcon[3] = {0.0, 0.0, 0.0};
-  const double sie = q[4] / rho;  // rho may be zero or subnormal where no floor acts
+  const double sie = div_any(q[4], rho);  // rho may be zero or subnormal where no floor acts
   const double u = (sie > sie_floor ? (sie > sie_max ? rho * sie_max : q[4]) : rho * sie_floor);
   const double P = smax(q[L::prs], 0.0);
   const double gamma1 = q[L::gm1];

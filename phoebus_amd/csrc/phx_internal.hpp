@@ -142,8 +142,8 @@ int check_params(phx_ctx *ctx, const phx_fluid_params *p);
 int check_block(phx_ctx *ctx, const phx_block *b, int recon);
 
 void launch_flux_ct(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s);
-// FluxCT's corner EMFs alone (the fused updates form the rewritten B fluxes from them)
-// the corner EMFs; dt given: also dt[0] = dt0, for kernels after it that lower it
+// FluxCT's corner EMFs alone (the fused updates form the rewritten B fluxes from them); dt
+// given: also dt[0] = dt0, for kernels after it that lower it
 void launch_ct_emf(const BlockGeom &bg, const FluxPtrs &flux, double *emf, hipStream_t s,
                    double *dt = nullptr, double dt0 = 0.0);
 // the corner EMFs and the sources of a curved MHD block (2-D, 3-D) in one launch

@@ -252,6 +252,7 @@ void launch_exchange_and_boundaries(phx_mesh *m, int st, hipStream_t s) {
   ctx->mark_end(s);
 }
 
+// the learned-bracket pass over the cells queued since the queue was last cleared
 void launch_c2p_queued(phx_mesh *m, int st, const char *name, hipStream_t s) {
   phx_pack *k = m->pack;
   m->ctx->mark_begin(name, s);

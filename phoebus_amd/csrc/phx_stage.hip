@@ -286,8 +286,8 @@ void launch_update_con2prim_entire(const phx_fluid_params &p, const BlockGeom &b
 
 // packs: the fused update over a work list of 3-D MHD blocks; dt from dt_dev when given
 // (a device-resident time step, so a captured graph needs no host value).  Every FMKS
-// block of a pack carries its cached geometry; the FMKS variant fits four waves per SIMD
-// (128 VGPRs) without spilling.
+// block of a pack carries its cached geometry; the FMKS variant is held to four waves per SIMD
+// (128 VGPRs, 17 of them spilled, 15 with FACE).
 // FACE: the first nf groups take the con2prim of the ghost cells in vf (work-list kind 6: what
 // the c2p fixup reads besides the interior) on U_{s+1}, cells that the update neither reads nor
 // writes: 524,288 cells and an 81,920-lane layer 108 us against 97 + 24.

@@ -18,8 +18,8 @@ import _oracle as O
 from phoebus_amd import _abi as A
 from phoebus_amd.api import BlockState, Pack, Phx, block, fluid_params
 from phoebus_amd.device import DeviceArray, synchronize
-from test_gpu_parity import (CASES, case_id, consumed_face_slices, geom_block, geom_params,
-                             oblock, oparams, random_block)
+from test_gpu_parity import (CASES, EVACUATED, case_id, consumed_face_slices, geom_block,
+                             geom_params, oblock, oparams, random_block)
 
 pytestmark = pytest.mark.gpu
 
@@ -98,6 +98,35 @@ def test_fast_curved_fluxes_at_the_bounds(phx, geom, mhd):
             for m in range(rf.shape[1]):
                 _flux_close(gf[d, m][sl], rf[d, m][sl], f"recon={recon} d={d} m={m}")
             _flux_close(gs[d][sl], rs[d][sl], f"face_sig d={d}")
+
+
+@pytest.mark.parametrize("geom", [A.GEOM_MINKOWSKI, A.GEOM_SPHERICAL_KS])
+@pytest.mark.parametrize("bounds", EVACUATED)
+def test_fast_fluxes_of_evacuated_zones(phx, bounds, geom):
+    """Zero, subnormal and tiny densities, energies and pressures beside ordinary ones, at the
+    block test's tolerance (a subnormal denominator must not become an infinity)."""
+    say(f"[gpu] fast fluxes of evacuated zones, bounds {bounds} geom {geom}")
+    rng = np.random.default_rng(12)
+    b = geom_block(3, (11, 9, 8), geom)
+    for mhd in (False, True):
+        prim = random_block(rng, b, mhd, 4.0 / 3.0, geom)
+        for v in (0, 4, prim.shape[0] - 2):  # rho, u, P
+            prim[v] = rng.choice([0.0, 5e-324, 1e-310, 2.3e-308, 1e-300, 1e-20, 1.0],
+                                 prim.shape[1:])
+        for recon in (A.RECON_CONSTANT, A.RECON_LINEAR):
+            p = geom_params(geom, gamma=4.0 / 3.0, mhd=mhd, recon=recon, riemann=A.RIEMANN_HLL,
+                            flux_arith=A.FLUX_ARITH_FAST, **EVACUATED[bounds])
+            rf, rs = O.calculate_fluxes(oparams(p), oblock(b), prim)
+            st = BlockState(p, b)
+            st.prim.upload(prim)
+            phx.calculate_fluxes(p, b, st.fields())
+            synchronize()
+            gf, gs = st.flux.get(), st.face_sig.get()
+            for d in range(3):
+                sl = consumed_face_slices(b, d)
+                for m in range(rf.shape[1]):
+                    _flux_close(gf[d, m][sl], rf[d, m][sl], f"mhd={mhd} recon={recon} d={d} m={m}")
+                _flux_close(gs[d][sl], rs[d][sl], f"mhd={mhd} recon={recon} face_sig d={d}")
 
 
 def test_fast_sweep_shapes_agree(phx):
